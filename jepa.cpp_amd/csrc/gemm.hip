@@ -25,6 +25,7 @@
 // loads with an LDS destination into an XOR-swizzled layout, several stages in flight.
 #include "kernels.h"
 #include "model.h"
+#include "gemm_dev.h"
 #include "lds_dma.h"
 #include "lanes.h"
 #include "quant_dev.h"
@@ -47,49 +48,8 @@ typedef unsigned int u4v __attribute__((ext_vector_type(4)));
 
 namespace {
 
-struct kargs {
-    const _Float16 * A;      // [N][K] weight codes (or f16 / f32 weights)
-    const uint16_t * Ad;     // W_Q32, W_Q40: f16 d [N][K/32]; W_Q4K: u32 (d | dmin << 16) [K/256][N]
-    const _Float16 * Amin;   // W_Q4K: [N][K/256][16] sub-block mins, each twice
-    const uint8_t * Asc;     // W_Q4K: [N][K/256][8] 6-bit sub-block scales
-    const _Float16 * B;      // [M][K] activation codes (or f16 / f32 activations)
-    const void * Bd;         // A_Q8_0: f16 d [M][K/32]; A_Q8_K: f32 d [M][K/256]
-    const _Float16 * Bsum;   // A_Q8_K: f16 bsums [M][K/16]
-    const float * bias;
-    int64_t M, N, K;
-    int tn, tm;              // workgroup tiles along N and M
-    int xa, xb;              // tiles per XCD block along N and M (0: plain order)
-    int split;               // K halves computed by separate workgroups (1 or 2; q8_0 / q4_0 / q4_K)
-    float * part;            // split: raw accumulators of every workgroup [split][tiles][BN*BM]
-    int * cnt;               // split: arrivals per tile (0 between launches)
-    gemm_epi ep;
-};
-
 __device__ __forceinline__ float h2f(uint16_t b) { return (float) __builtin_bit_cast(_Float16, b); }
 __device__ __forceinline__ uint16_t f2hbits(float f) { return __builtin_bit_cast(uint16_t, (_Float16) f); }
-
-// GELU(x) = 0.5 x (1 + erf(x / sqrt 2)) = x Phi(x) (ggml_vec_gelu_erf_f32, reference
-// docs/ggml-notes.md:291-292), Phi the standard normal CDF, from its tail h(t) = Phi(-t), t = |x|:
-//   Phi(x) = 1 - h(t) for x >= 0, h(t) for x < 0,   h(t) = 2^Q(min(t, 5.5)), Q of degree 8 with Q(0) = -1
-// One polynomial and one hardware exp2 per value, no branch: 14 VALU ops where erf's two-piece form
-// (both pieces evaluated, one selected) took 25. Coefficients from fit_gelu.py (fitted with weight h,
-// so the absolute error of Phi is minimised; Q(0) = -1 gives Phi(0) = 1/2 exactly): the float32
-// evaluation stays within 1.5 units of 2^-24 of Phi (2.5 with exp2 two units off), about the accuracy
-// of the libm erff form. At t = 5.5, h = 1.9e-8 < 2^-25, so 1 - h is 1.0f and GELU(x) = x beyond.
-__device__ __forceinline__ float gelu_erf(float x) {
-    const float t = fminf(fabsf(x), 5.5f);
-    float q = -2.248140163e-06f;
-    q = fmaf(q, t, 3.268636283e-05f);
-    q = fmaf(q, t, -1.560558158e-04f);
-    q = fmaf(q, t, -2.054840443e-04f);
-    q = fmaf(q, t, 7.147170603e-03f);
-    q = fmaf(q, t, -5.254988000e-02f);
-    q = fmaf(q, t, -4.591920078e-01f);
-    q = fmaf(q, t, -1.151106834e+00f);
-    q = fmaf(q, t, -1.0f);
-    const float h = __builtin_amdgcn_exp2f(q);
-    return __fmul_rn(x, x >= 0.0f ? __fsub_rn(1.0f, h) : h);
-}
 
 // The residual epilogue with the row's current values x already loaded: x + (t + bias) * ls
 // (bias b and layer scale v already loaded: zero / unused when absent)
@@ -114,82 +74,6 @@ __device__ __forceinline__ void f32out4(const kargs & a, int64_t m, int64_t n, f
     const int64_t item = m / ep.rin, rr = m - item * ep.rin;
     const int64_t row = item * ep.rout + ep.pre + rr;
     *(float4 *) (ep.y + row * ep.ldy + n) = make_float4(t[0], t[1], t[2], t[3]);
-}
-
-__device__ __forceinline__ int perm16(int64_t tok) {
-    // position of token `tok` inside its 16-token group of V^T (see attention.hip)
-    const int key = (int) (tok & 15);
-    const int gg = (key >> 2) & 1, s = (key & 3) + 4 * (key >> 3);
-    return (int) (tok & ~(int64_t) 15) + 8 * gg + s;
-}
-
-// Epilogue of 4 consecutive features n..n+3 of row m (values t[] = raw accumulators).
-template <int EPI>
-__device__ __forceinline__ void epi4(const kargs & a, int64_t m, int64_t n, float t[4]) {
-    const gemm_epi & ep = a.ep;
-    if (a.bias) {
-        const float4 b = *(const float4 *) (a.bias + n);
-        t[0] = __fadd_rn(t[0], b.x); t[1] = __fadd_rn(t[1], b.y); t[2] = __fadd_rn(t[2], b.z); t[3] = __fadd_rn(t[3], b.w);
-    }
-    if constexpr (EPI == EPI_F32) {
-        if (ep.addvec) {
-            const float4 v = *(const float4 *) (ep.addvec + n);
-            t[0] = __fadd_rn(t[0], v.x); t[1] = __fadd_rn(t[1], v.y); t[2] = __fadd_rn(t[2], v.z); t[3] = __fadd_rn(t[3], v.w);
-        }
-        const int64_t item = m / ep.rin, r = m - item * ep.rin;
-        const int64_t row = item * ep.rout + ep.pre + r;
-        if (ep.addrows) {
-            const float4 v = *(const float4 *) (ep.addrows + (ep.pre + r) * ep.ldy + n);
-            t[0] = __fadd_rn(t[0], v.x); t[1] = __fadd_rn(t[1], v.y); t[2] = __fadd_rn(t[2], v.z); t[3] = __fadd_rn(t[3], v.w);
-        }
-        *(float4 *) (ep.y + row * ep.ldy + n) = make_float4(t[0], t[1], t[2], t[3]);
-    } else if constexpr (EPI == EPI_RESID) {
-        if (ep.ls) {
-            const float4 v = *(const float4 *) (ep.ls + n);
-            t[0] = __fmul_rn(t[0], v.x); t[1] = __fmul_rn(t[1], v.y); t[2] = __fmul_rn(t[2], v.z); t[3] = __fmul_rn(t[3], v.w);
-        }
-        float4 * px = (float4 *) (ep.y + m * ep.ldy + n);
-        float4 x = *px;
-        x.x = __fadd_rn(x.x, t[0]); x.y = __fadd_rn(x.y, t[1]); x.z = __fadd_rn(x.z, t[2]); x.w = __fadd_rn(x.w, t[3]);
-        *px = x;
-    } else if constexpr (EPI == EPI_GELU_F32) {
-        *(float4 *) (ep.y + m * ep.ldy + n) = make_float4(gelu_erf(t[0]), gelu_erf(t[1]), gelu_erf(t[2]), gelu_erf(t[3]));
-    } else if constexpr (EPI == EPI_GELU_F16) {
-        _Float16 * o = (_Float16 *) ep.oh + m * ep.ldy + n;
-        typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-        h4 v = {(_Float16) gelu_erf(t[0]), (_Float16) gelu_erf(t[1]), (_Float16) gelu_erf(t[2]), (_Float16) gelu_erf(t[3])};
-        *(h4 *) o = v;
-    } else if constexpr (EPI == EPI_QKV) {
-        const int D = ep.D, hd = ep.hd, hds = ep.hds ? ep.hds : hd;
-        const int64_t ng = n + ep.col0;        // column of the [q | k | v] layout (the bias above is this launch's)
-        const int which = (int) (ng / D);
-        const int nn = (int) (ng - (int64_t) which * D);
-        const int h = nn / hd, d0 = nn - h * hd;
-        const int64_t item = m / ep.R, tok = m - item * ep.R;
-        const int64_t head = item * ep.n_head + h;
-        if (which < 2) {
-            float o[4];
-            if (ep.rope_c) {
-                // out = x*C + swap(x)*S' (reference src/rope3d.cpp:136-164): two products, one add
-                const float4 c = *(const float4 *) (ep.rope_c + tok * hd + d0);
-                const float4 s = *(const float4 *) (ep.rope_s + tok * hd + d0);
-                o[0] = __fadd_rn(__fmul_rn(t[0], c.x), __fmul_rn(t[1], s.x));
-                o[1] = __fadd_rn(__fmul_rn(t[1], c.y), __fmul_rn(t[0], s.y));
-                o[2] = __fadd_rn(__fmul_rn(t[2], c.z), __fmul_rn(t[3], s.z));
-                o[3] = __fadd_rn(__fmul_rn(t[3], c.w), __fmul_rn(t[2], s.w));
-            } else {
-                o[0] = t[0]; o[1] = t[1]; o[2] = t[2]; o[3] = t[3];
-            }
-            typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-            h4 v = {(_Float16) o[0], (_Float16) o[1], (_Float16) o[2], (_Float16) o[3]};
-            _Float16 * dst = (_Float16 *) (which == 0 ? ep.q : ep.k) + (head * ep.R_pad + tok) * hds + d0;
-            *(h4 *) dst = v;
-        } else {
-            _Float16 * vt = (_Float16 *) ep.vt + head * hds * ep.R_pad;
-            const int p = perm16(tok);
-            for (int e = 0; e < 4; e++) vt[(int64_t) (d0 + e) * ep.R_pad + p] = (_Float16) t[e];
-        }
-    }
 }
 
 // Stage barrier: wait until at most N_ of this wave's HBM->LDS copies are outstanding and its LDS reads
@@ -1426,120 +1310,6 @@ __global__ __launch_bounds__(64 * WN * WM, 1) void k_gemm_mfma(const void * pA, 
     }
 }
 
-// f32 weights x f32 activations (hfvit patch embedding and f32 files): VALU FMA on tiles of 16 tokens x
-// 32 features, so that even a one-image patch embedding (196 x 384 outputs) runs on 156 workgroups.
-// A workgroup stages up to F32_KC columns of its 16 activation rows and 32 weight rows in LDS at once,
-// row-major as loaded (16-byte stores; rows padded by 4 floats so that the rows one read touches fall
-// on different banks), then each of its sixteen waves (four per SIMD, to hide the LDS and FMA
-// latencies) sums one slice of those columns, four columns at a time: a lane holds 2 tokens x 4
-// consecutive features, six 16-byte LDS reads per 32 FMAs. The partial sums meet in LDS and are added
-// in wave order; a K longer than F32_KC runs several such
-// chunks, each chunk's total added to the running sum.
-constexpr int F32_KC = 768, F32_LD = F32_KC + 4;
-constexpr int F32_NW = 16;                              // waves per workgroup, one K slice each
-template <int EPI>
-__global__ __launch_bounds__(64 * F32_NW) void k_gemm_f32(kargs a) {
-    __shared__ __attribute__((aligned(16))) float sX[16][F32_LD];
-    __shared__ __attribute__((aligned(16))) float sW[32][F32_LD];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int64_t n0 = (int64_t) blockIdx.x * 32, m0 = (int64_t) blockIdx.y * 16;
-    const float * W = (const float *) a.A;
-    const float * X = (const float *) a.B;
-    const int tg = lane >> 3, fg = lane & 7;            // tokens 2 tg, 2 tg + 1; features 4 fg .. 4 fg + 3
-    const bool al = (a.K & 3) == 0 && (((uintptr_t) X | (uintptr_t) W) & 15) == 0;   // rows 16-byte aligned
-    float tot[2][4] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
-    float * red = &sW[0][0];                            // [F32_NW - 1][64][8] partials of waves 1.. (reuses sW)
-    // one 4-column piece of row r of a (rows past `rows`, columns past kc read as 0)
-    auto piece = [&](const float * base, int64_t row, int64_t rows, int64_t k0, int kk, int kc) {
-        float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        if (row < rows) {
-            const float * src = base + row * a.K + k0 + kk;
-            if (kk + 4 <= kc && al) v = *(const float4 *) src;
-            else { v.x = src[0]; if (kk + 1 < kc) v.y = src[1]; if (kk + 2 < kc) v.z = src[2]; if (kk + 3 < kc) v.w = src[3]; }
-        }
-        return v;
-    };
-    for (int64_t k0 = 0; k0 < a.K; k0 += F32_KC) {
-        const int kc = (int) (a.K - k0 < F32_KC ? a.K - k0 : F32_KC);
-        const int kc4 = (kc + 3) & ~3;                  // columns staged: kc rounded up to 4 (zeros past kc)
-        __syncthreads();                                // the previous chunk's reads (and reduction) are done
-        // every load is issued before the LDS stores (a store between two loads would hold the second
-        // back: the compiler cannot tell the rows from LDS); 9 pieces per thread, one round trip
-        constexpr int PT = 16 * (F32_KC / 4) / (64 * F32_NW);   // pieces per thread per 16 rows
-        float4 v[3][PT];
-#pragma unroll
-        for (int b = 0; b < 3; b++)                     // rows 0-15 of X, then 0-15 and 16-31 of W
-#pragma unroll
-            for (int i = 0; i < PT; i++) {
-                const int c = tid + 64 * F32_NW * i, r = c / (F32_KC / 4), kk = 4 * (c % (F32_KC / 4));
-                v[b][i] = kk < kc ? (b == 0 ? piece(X, m0 + r, a.M, k0, kk, kc) : piece(W, n0 + 16 * (b - 1) + r, a.N, k0, kk, kc))
-                                  : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            }
-#pragma unroll
-        for (int b = 0; b < 3; b++)
-#pragma unroll
-            for (int i = 0; i < PT; i++) {
-                const int c = tid + 64 * F32_NW * i, r = c / (F32_KC / 4), kk = 4 * (c % (F32_KC / 4));
-                if (kk < kc) *(float4 *) (b == 0 ? &sX[r][kk] : &sW[16 * (b - 1) + r][kk]) = v[b][i];
-            }
-        __syncthreads();
-        const int q = ((kc4 / 4 + F32_NW - 1) / F32_NW) * 4;   // columns per wave, a multiple of 4
-        const int kb = wave * q, ke = kb + q < kc4 ? kb + q : kc4;
-        float acc[2][4] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
-        for (int k = kb; k < ke; k += 4) {
-            const float4 x0 = *(const float4 *) &sX[2 * tg][k], x1 = *(const float4 *) &sX[2 * tg + 1][k];
-            float4 w[4];
-#pragma unroll
-            for (int e = 0; e < 4; e++) w[e] = *(const float4 *) &sW[4 * fg + e][k];
-            const float xa[2][4] = {{x0.x, x0.y, x0.z, x0.w}, {x1.x, x1.y, x1.z, x1.w}};
-#pragma unroll
-            for (int j = 0; j < 4; j++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const float wv = j == 0 ? w[e].x : j == 1 ? w[e].y : j == 2 ? w[e].z : w[e].w;
-                    acc[0][e] = fmaf(xa[0][j], wv, acc[0][e]);
-                    acc[1][e] = fmaf(xa[1][j], wv, acc[1][e]);
-                }
-        }
-        __syncthreads();                                // every wave is past its reads of sW
-        if (wave > 0) {
-#pragma unroll
-            for (int i = 0; i < 2; i++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) red[((wave - 1) * 64 + lane) * 8 + 4 * i + e] = acc[i][e];
-        }
-        __syncthreads();
-        if (wave == 0) {
-#pragma unroll
-            for (int i = 0; i < 2; i++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    float v = acc[i][e];
-                    for (int w = 0; w < F32_NW - 1; w++) v = __fadd_rn(v, red[(w * 64 + lane) * 8 + 4 * i + e]);
-                    tot[i][e] = k0 == 0 ? v : __fadd_rn(tot[i][e], v);
-                }
-        }
-    }
-    if (wave == 0) {
-#pragma unroll
-        for (int i = 0; i < 2; i++) {
-            const int64_t m = m0 + 2 * tg + i, n = n0 + 4 * fg;
-            if (m < a.M && n < a.N) epi4<EPI>(a, m, n, tot[i]);
-        }
-    }
-}
-
-// f32 fused-qkv rows -> Q, K (RoPE'd) and V^T through the same epilogue the QKV GEMM runs
-__global__ void k_qkv_split(kargs a, const float * __restrict__ qkv) {
-    const int64_t id = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t groups = a.N / 4;
-    if (id >= a.M * groups) return;
-    const int64_t m = id / groups, n = (id % groups) * 4;
-    const float4 v = *(const float4 *) (qkv + m * a.N + n);
-    float t[4] = {v.x, v.y, v.z, v.w};
-    epi4<EPI_QKV>(a, m, n, t);
-}
-
 struct tile_cfg { int wn, wm, ti, tj; };
 // eight-wave workgroup tiles (BN x BM): 256x128, 192x128, 128x128 (two wave shapes), 64x128, 128x64,
 // 256x64 (two wave shapes; the second, one weight tile and two token tiles per wave, only for the
@@ -1771,14 +1541,7 @@ void launch_gemm(const dev_linear & W, const act_view & X, int64_t M, const gemm
     }
     if (a.ep.kind == EPI_F32 && a.ep.rin <= 0) { a.ep.rin = M; a.ep.rout = M; a.ep.pre = 0; }   // identity row map
     if (W.fmt == W_F32) {
-        dim3 grid((unsigned) ((a.N + 31) / 32), (unsigned) ((M + 15) / 16));
-        switch (ep.kind) {
-            case EPI_F32:      k_gemm_f32<EPI_F32><<<grid, 64 * F32_NW, 0, s>>>(a); break;
-            case EPI_RESID:    k_gemm_f32<EPI_RESID><<<grid, 64 * F32_NW, 0, s>>>(a); break;
-            case EPI_GELU_F32: k_gemm_f32<EPI_GELU_F32><<<grid, 64 * F32_NW, 0, s>>>(a); break;
-            case EPI_QKV:      k_gemm_f32<EPI_QKV><<<grid, 64 * F32_NW, 0, s>>>(a); break;
-            default: jepa_log("jepa: internal error: epilogue %d has no f32 GEMM\n", ep.kind); break;
-        }
+        launch_gemm_f32(W, X, M, a.ep, s);
         return;
     }
     switch (W.fmt) {
@@ -1799,12 +1562,4 @@ int gemm_force_tile(int index) {
     if (index >= (int) (sizeof(k_tiles) / sizeof(k_tiles[0]))) return -1;
     g_force_tile.store(index < 0 ? -1 : index);
     return 0;
-}
-
-void launch_qkv_split(const float * qkv, int64_t M, int64_t N, const gemm_epi & ep, hipStream_t s) {
-    kargs a{};
-    a.M = M; a.N = N; a.K = 0;
-    a.ep = ep;
-    const int64_t total = M * (N / 4);
-    if (total > 0) k_qkv_split<<<(unsigned) ((total + 255) / 256), 256, 0, s>>>(a, qkv);
 }

@@ -68,6 +68,8 @@ void gemm_split_ws_size(int64_t max_rows, int64_t * part_floats, int64_t * cnt_n
 // Y = X W^T (+ epilogue). M = rows of X. Without split scratch every tile is one workgroup.
 void launch_gemm(const dev_linear & W, const act_view & X, int64_t M, const gemm_epi & ep, hipStream_t s,
                  const gemm_split_ws * sw = nullptr);
+// the same for f32 weights and activations (launch_gemm's W_F32 case; gemm_f32.hip)
+void launch_gemm_f32(const dev_linear & W, const act_view & X, int64_t M, const gemm_epi & ep, hipStream_t s);
 // K halves the int8 / 4-bit GEMM of this weight format and shape runs in (1 or 2); depends on N and K
 // only, so that the summation order of an output never depends on the number of rows (f16 weights:
 // chosen per launch from the tile count, 1 here)

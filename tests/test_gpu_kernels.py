@@ -176,6 +176,28 @@ def test_matmul_full_m2048_q8_0(jlib, oracle):
     np.testing.assert_array_equal(host(y).view(np.uint32), want.view(np.uint32))
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 128, 8), (31, 128, 40), (33, 96, 128), (64, 36, 136), (197, 384, 768), (40, 1280, 584)])
+def test_matmul_f32(jlib, M, N, K):
+    """f32 weights on the f32 matrix instruction (32 x 32 tiles, K in chunks of 16 columns dealt to eight waves,
+    four accumulators each): ragged rows, features and column chunks, waves without a chunk. Against 64 bits,
+    within the bound of its sums: at most n roundings on the way of any product, each 2^-24 of the sum of the
+    products' magnitudes at most; n = the products of one accumulator (4 per chunk of a wave), then 2 + 7
+    additions and the bias."""
+    rng = np.random.default_rng(M + N + K)
+    w = rng.standard_normal((N, K)).astype(np.float32)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    bias = rng.standard_normal(N).astype(np.float32)
+    dw, dx, db = dev(w), dev(x), dev(bias)
+    y = torch.full((M, N), float("nan"), dtype=torch.float32, device="cuda")
+    torch.cuda.synchronize()
+    rc = jlib.lib().jepa_amd_matmul(0, gguf.GGML_F32, dw.data_ptr(), N, K, db.data_ptr(), dx.data_ptr(), M, y.data_ptr(), 1, None)
+    assert rc == 0, jlib.error_text()
+    w64, x64 = w.astype(np.float64), x.astype(np.float64)
+    n = 4 * -(-(-(-K // 16)) // 8) + 2 + 7 + 1
+    bound = n * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64).T + np.abs(bias))
+    assert (np.abs(host(y) - (x64 @ w64.T + bias)) <= bound).all()
+
+
 def _q8k_blocks(raw, n_rows, n_cols):
     """ggml block_q8_K bytes -> (d f32 [rows][nb], codes int8 [rows][n_cols], bsums int16 [rows][nb*16])"""
     b = raw.reshape(n_rows, n_cols // 256, 292)
