@@ -8,7 +8,12 @@
 //              LN2 -> codes | up GEMM + bias + GELU(erf) -> codes of the down GEMM's input
 //              down GEMM + bias (* ls2) + residual into x
 //   final LN -> f32 output rows
-// The whole sequence for one input shape is captured once into a hipGraph and replayed.
+// Everything between the first and the last kernel touches only the workspace and the weights: for one
+// input shape it is captured once into a hipGraph and replayed. The patchify launch, which reads the
+// caller's input, and the final LN, which writes the caller's output, go to the stream around the replay,
+// so that a call with buffers not seen before costs the same as a repeated one (a graph that held the
+// pointers was captured and instantiated again for each new pair: ~10 us of host time per kernel,
+// 1.7 ms on the 171 kernels of ViT-L).
 #include "forward.h"
 #include "rope3d.h"
 
@@ -283,8 +288,30 @@ bool ensure_workspace(jepa_context * ctx, int n_items, int n_chans, int n_frames
     return true;
 }
 
-// Enqueue the forward of the workspace's shape on ctx->stream. in: NCTHW f32 of n_items; out: [rows][D].
-void enqueue_forward(jepa_context * ctx, const float * in, float * out, float * trace, ktimer & kt) {
+// The forward of the workspace's shape, enqueued on ctx->stream in three parts: the input (NCTHW f32 of
+// n_items) into patch rows, the encoder on the workspace's buffers, the output rows [rows][D].
+void enqueue_input(jepa_context * ctx, const float * in, ktimer & kt) {
+    const jepa_model * m = ctx->model;
+    const fwd_workspace & w = *ctx->ws;
+    const dev_linear & pe = w.image_path ? m->patch_img : m->patch;
+    kt.run("patchify", [&] {
+        launch_patchify(in, w.patches, pe.fmt != W_F32, w.n_items, w.n_chans, w.n_frames, w.height, w.width, m->hp.enc.patch_size,
+                        w.tubelet, w.video, ctx->stream);
+    });
+}
+
+void enqueue_output(jepa_context * ctx, float * out, ktimer & kt) {
+    const jepa_model * m = ctx->model;
+    const enc_hparams & e = m->hp.enc;
+    const fwd_workspace & w = *ctx->ws;
+    act_view o;
+    o.fmt = A_F32; o.q = out; o.ld = e.embed_dim;
+    kt.run("layernorm", [&] {
+        launch_rownorm_quant(w.x, w.n_items * w.R, e.embed_dim, m->norm_w, m->norm_b, e.ln_eps, true, o, ctx->stream);
+    });
+}
+
+void enqueue_encoder(jepa_context * ctx, float * trace, ktimer & kt) {
     const jepa_model * m = ctx->model;
     const enc_hparams & e = m->hp.enc;
     fwd_workspace & w = *ctx->ws;
@@ -292,10 +319,6 @@ void enqueue_forward(jepa_context * ctx, const float * in, float * out, float * 
     const int64_t n_items = w.n_items, R = w.R, D = e.embed_dim, rows = n_items * R;
     const dev_linear & pe = w.image_path ? m->patch_img : m->patch;
 
-    kt.run("patchify", [&] {
-        launch_patchify(in, w.patches, pe.fmt != W_F32, n_items, w.n_chans, w.n_frames, w.height, w.width, e.patch_size, w.tubelet,
-                        w.video, s);
-    });
     {
         act_view pa;
         pa.fmt = pe.act();
@@ -325,9 +348,6 @@ void enqueue_forward(jepa_context * ctx, const float * in, float * out, float * 
         enqueue_block(bs, m->layers[(size_t) l], w, n_items, R, w.rope_c, w.rope_s, n_prefix, slot_rows, s, kt);
         if (trace) launch_copy_f32(w.x, trace + (int64_t) (l + 1) * rows * D, rows * D, s);
     }
-    act_view o;
-    o.fmt = A_F32; o.q = out; o.ld = D;
-    kt.run("layernorm", [&] { launch_rownorm_quant(w.x, rows, D, m->norm_w, m->norm_b, e.ln_eps, true, o, s); });
 }
 
 bool check_supported(const jepa_model * m) {
@@ -442,16 +462,15 @@ int64_t encode_device(jepa_context * ctx, const float * in_dev, int n_batch, int
         ktimer kt{ctx};
         hipEventRecord(ctx->ev0, ctx->stream);
         if (trace_dev || ctx->kernel_timing || !ctx->use_graph) {
-            enqueue_forward(ctx, src, dst, trace_dev, kt);
+            enqueue_input(ctx, src, kt);
+            enqueue_encoder(ctx, trace_dev, kt);
         } else {
-            if (!w.graph_ok || w.g_in != src || w.g_out != dst) {
+            if (!w.graph_ok) {
                 std::lock_guard<std::recursive_mutex> lk(jepa_hip_mutex());
-                if (w.exec) { hipGraphExecDestroy(w.exec); w.exec = nullptr; }
-                w.graph_ok = false;
                 hipGraph_t graph = nullptr;
                 bool cap = hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal) == hipSuccess;
                 if (cap) {
-                    enqueue_forward(ctx, src, dst, nullptr, kt);
+                    enqueue_encoder(ctx, nullptr, kt);
                     cap = hipStreamEndCapture(ctx->stream, &graph) == hipSuccess && graph &&
                           hipGraphInstantiate(&w.exec, graph, nullptr, nullptr, 0) == hipSuccess;
                     if (graph) hipGraphDestroy(graph);
@@ -460,18 +479,18 @@ int64_t encode_device(jepa_context * ctx, const float * in_dev, int n_batch, int
                     // capture is an optimisation: fall back to direct launches (same kernels)
                     hipGetLastError();
                     ctx->use_graph = false;
-                    enqueue_forward(ctx, src, dst, nullptr, kt);
-                } else {
-                    w.graph_ok = true;
-                    w.g_in = src;
-                    w.g_out = dst;
                 }
+                w.graph_ok = cap;
             }
-            if (w.graph_ok && hipGraphLaunch(w.exec, ctx->stream) != hipSuccess) {
+            enqueue_input(ctx, src, kt);
+            if (!w.graph_ok) {
+                enqueue_encoder(ctx, nullptr, kt);
+            } else if (hipGraphLaunch(w.exec, ctx->stream) != hipSuccess) {
                 jepa_log("jepa: hipGraphLaunch failed\n");
                 return -1;
             }
         }
+        enqueue_output(ctx, dst, kt);
         hipEventRecord(ctx->ev1, ctx->stream);
         const hipError_t st = hipEventSynchronize(ctx->ev1);
         if (st != hipSuccess) { jepa_log("jepa: forward failed on device %d: %s\n", ctx->device, hipGetErrorString(st)); return -1; }

@@ -33,7 +33,6 @@ struct fwd_workspace {
     act_view actC;
     // graph
     hipGraphExec_t exec = nullptr;
-    const float * g_in = nullptr; float * g_out = nullptr;
     bool graph_ok = false;
 
     void release() {
