@@ -407,8 +407,9 @@ extern "C" int jepa_amd_preprocess_frames_device(int device, const jepa_preproce
     }
     dev_scope d(device);
     if (!d.ok) return -1;
-    void * scratch = d.alloc(preprocess_scratch_bytes(p, g, n_frames, h, w));
-    if (!scratch) return -1;
+    const bool tiled = preprocess_tiled(p, g, n_frames, h, w);
+    void * scratch = tiled ? nullptr : d.alloc(preprocess_scratch_bytes(p, g, n_frames, h, w));
+    if (!tiled && !scratch) return -1;
     if (!launch_preprocess(p, g, frames, n_frames, h, w, out, scratch, d.s)) {
         jepa_log("jepa: jepa_amd_preprocess_frames_device: launch failed\n");
         return -1;
@@ -429,7 +430,8 @@ extern "C" int jepa_amd_preprocess_frames_device_noalloc(int device, const jepa_
                  (long long) need);
         return -1;
     }
-    const size_t bytes = preprocess_scratch_bytes(p, g, n_frames, h, w);
+    size_t bytes = preprocess_scratch_bound(p, g, n_frames, h, w);
+    if (bytes > PRE_NOALLOC_SCRATCH_BYTES) bytes = preprocess_scratch_bytes(p, g, n_frames, h, w);
     if (bytes > PRE_NOALLOC_SCRATCH_BYTES) {
         jepa_log("jepa: jepa_amd_preprocess_frames_device_noalloc: %d frames of %dx%d need %.1f MiB of scratch, over the %zu MiB "
                  "this entry point has (use jepa_amd_preprocess_frames_device, or fewer frames per call)\n",
@@ -444,7 +446,7 @@ extern "C" int jepa_amd_preprocess_frames_device_noalloc(int device, const jepa_
         return -1;
     }
     int rc = -1;
-    void * scratch = preprocess_static_scratch(device);
+    void * scratch = preprocess_static_scratch(device);   // (not used by the tiled kernel)
     if (scratch) {
         hipStream_t s = (hipStream_t) stream;
         if (!launch_preprocess(p, g, frames, n_frames, h, w, out, scratch, s)) {

@@ -29,34 +29,6 @@
 
 namespace {
 
-// the two antialias filters, each with its radius at scale 1
-struct aa_filter {
-    double radius;
-    double (*at)(double);
-};
-
-double triangle_at(double x) {
-    const double d = std::fabs(x);
-    return d < 1.0 ? 1.0 - d : 0.0;
-}
-
-// Keys (1981) cubic convolution, a = -0.5, in the nested form torch evaluates (the weights must be
-// the same doubles for the int16 rounding to agree): inner piece ((a+2)|x| - (a+3))|x|^2 + 1,
-// outer piece ((a|x| - 5a)|x| + 8a)|x| - 4a
-double keys_at(double x) {
-    constexpr double a = -0.5;
-    const double d = std::fabs(x);
-    if (d >= 2.0) return 0.0;
-    if (d >= 1.0) return ((a * d - 5.0 * a) * d + 8.0 * a) * d - 4.0 * a;
-    return ((a + 2.0) * d - (a + 3.0)) * d * d + 1.0;
-}
-
-// round half away from zero the way the method writes it, (int)(0.5 + |v|) with the sign put back
-int16_t round_tap(double v) {
-    const int mag = (int) (0.5 + std::fabs(v));
-    return (int16_t) (v < 0.0 ? -mag : mag);
-}
-
 uint8_t settle(int32_t acc, int shift) {
     const int32_t v = acc >> shift;
     return (uint8_t) std::min<int32_t>(255, std::max<int32_t>(0, v));
@@ -99,30 +71,45 @@ void resample_cols(const resample_axis & ax, const uint8_t * src, size_t len, ui
 
 }  // namespace
 
+int axis_shift_of_peak(double peak) {
+    for (int s = 0; s < 22; s++)
+        if ((int) (0.5 + peak * (double) (1 << (s + 1))) >= (1 << 15)) return s;
+    return 22;
+}
+
+int axis_shift(const axis_filter & f) {
+    double peak = 0.0;
+    for (int o = 0; o < f.n_out; o++) {
+        int first, end;
+        const double centre = axis_window(f, o, first, end);
+        double total = 0.0, top = 0.0;
+        for (int x = first; x < end; x++) {
+            const double v = axis_weight(f, x, centre);
+            total += v;
+            top = std::max(top, v);
+        }
+        if (total != 0.0) peak = std::max(peak, top / total);
+    }
+    return axis_shift_of_peak(peak);
+}
+
 resample_axis resample_axis_for(int n_in, int n_out, int resample) {
     resample_axis ax;
     if (n_in <= 0 || n_out <= 0) return ax;
     ax.n_in = n_in;
     ax.n_out = n_out;
-    const aa_filter f = resample == JEPA_RESAMPLE_BICUBIC ? aa_filter{2.0, keys_at} : aa_filter{1.0, triangle_at};
-    const double scale = (double) n_in / (double) n_out;
-    const double stretch = std::max(scale, 1.0);        // the filter widens only when shrinking
-    const double reach = f.radius * stretch;
-    const double step = 1.0 / stretch;
+    const axis_filter f = axis_filter_for(n_in, n_out, resample);
     ax.lo.resize((size_t) n_out);
     ax.beg.assign(1, 0);
     std::vector<double> weight;
     double peak = 0.0;
     for (int o = 0; o < n_out; o++) {
-        const double centre = scale * (o + 0.5);
-        // inputs whose window rounds into [centre - reach, centre + reach), clipped to the image (in
-        // double before the conversion, so that a very wide input cannot push it past INT_MAX)
-        const int first = (int) std::max(0.0, centre - reach + 0.5);
-        const int end = (int) std::min((double) n_in, centre + reach + 0.5);
+        int first, end;
+        const double centre = axis_window(f, o, first, end);
         const size_t row0 = weight.size();
         double total = 0.0;
         for (int x = first; x < end; x++) {
-            const double v = f.at((x - centre + 0.5) * step);
+            const double v = axis_weight(f, x, centre);
             weight.push_back(v);
             total += v;
         }
@@ -134,11 +121,7 @@ resample_axis resample_axis_for(int n_in, int n_out, int resample) {
         ax.lo[(size_t) o] = first;
         ax.beg.push_back((int32_t) weight.size());
     }
-    // shift: the first s in 0..21 whose next step would round the peak weight to 2^15 or more,
-    // else 22
-    ax.shift = 22;
-    for (int s = 0; s < 22; s++)
-        if ((int) (0.5 + peak * (double) (1 << (s + 1))) >= (1 << 15)) { ax.shift = s; break; }
+    ax.shift = axis_shift_of_peak(peak);
     ax.taps.resize(weight.size());
     const double unit = (double) (1 << ax.shift);
     for (size_t t = 0; t < weight.size(); t++) ax.taps[t] = round_tap(weight[t] * unit);

@@ -718,3 +718,26 @@ def test_preprocess_device_equals_host(jlib, hw, kw):
     assert (oh.value, ow.value) == want.shape[2:]
     got = host(out).reshape(want.shape)
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), f"{int((got != want).sum())} values differ"
+
+
+# the tile kernel: one to several groups of taps (reductions 0.5 to 9), ragged crops and sizes, images smaller than
+# the crop (zero padding), odd base addresses, few frames (short tiles); a reduction past its LDS takes the two kernels
+@pytest.mark.parametrize("resample", [0, 1])
+@pytest.mark.parametrize("T,h,w,short,crop", [
+    (1, 64, 64, 64, 64), (2, 96, 131, 224, 224), (1, 231, 517, 256, 225), (3, 333, 250, 64, 96), (40, 120, 161, 66, 66), (1, 719, 1283, 292, 256),
+    (2, 1080, 1921, 224, 224), (1, 1100, 1501, 120, 112), (1, 37, 2500, 32, 48), (1, 900, 1000, 30, 32),
+])
+def test_preprocess_tile_kernel_equals_host(jlib, T, h, w, short, crop, resample):
+    rng = np.random.default_rng(T * h + w)
+    frames = rng.integers(0, 256, (T, h, w, 3), dtype=np.uint8)
+    p = _pre_params(jlib, resize_short=short, crop=crop, resample=resample)
+    want = jlib.preprocess_frames(p, list(frames)).reshape(-1)
+    for lead in (0, 1, 3):      # the frames' address modulo four
+        d = torch.zeros(frames.size + lead, dtype=torch.uint8, device="cuda")
+        d[lead:] = torch.from_numpy(frames.reshape(-1)).cuda()
+        out = torch.full((want.size,), float("nan"), device="cuda")
+        torch.cuda.synchronize()
+        rc = jlib.lib().jepa_amd_preprocess_frames_device(0, C.byref(p), d.data_ptr() + lead, T, h, w, out.data_ptr(), out.numel(), None, None)
+        assert rc == 0, jlib.error_text()
+        got = host(out)
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), f"lead {lead}: {int((got != want).sum())} values differ"
