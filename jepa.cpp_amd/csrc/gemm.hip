@@ -1315,9 +1315,9 @@ struct tile_cfg { int wn, wm, ti, tj; };
 // 256x64 (two wave shapes; the second, one weight tile and two token tiles per wave, only for the
 // 256-feature q8_K epilogue)
 constexpr tile_cfg k_tiles[] = {{4, 2, 2, 2}, {2, 4, 3, 1}, {2, 4, 2, 1}, {4, 2, 1, 2}, {2, 4, 1, 1}, {4, 2, 1, 1}, {4, 2, 2, 1},
-                                {8, 1, 1, 2}, {4, 2, 3, 1}};
+                                {8, 1, 1, 2}, {4, 2, 3, 1}, {2, 2, 1, 1}};
 // relative efficiency of one workgroup tile (larger tiles re-read less from L2 and LDS)
-constexpr double k_tile_eff[] = {1.0, 0.95, 0.85, 0.85, 0.65, 0.66, 0.8, 0.8, 0.9};
+constexpr double k_tile_eff[] = {1.0, 0.95, 0.85, 0.85, 0.65, 0.66, 0.8, 0.8, 0.9, 0.54};
 
 std::atomic<int> g_force_tile{-1};
 std::atomic<int> g_force_split{-1};
@@ -1340,7 +1340,7 @@ int cu_count() {
 // per SIMD, at most two MFMA tiles per wave. The 384x64 tile (for N = 3072: 256 tiles at M = 2048, the
 // role the 192x128 tile has for int8 weights) fits three LDS stages only with 4-bit weights.
 bool tile_ok(int wf, int c) {
-    if (wf == W_Q4K) return c == 2 || c == 3 || c == 5 || c == 6 || c == 7;
+    if (wf == W_Q4K) return c == 2 || c == 3 || c == 5 || c == 6 || c == 7 || c == 9;
     if (wf == W_Q40) return c != 1 && c != 4;
     return c != 8;
 }
@@ -1407,6 +1407,7 @@ void launch_tiles(int c, const kargs & a, hipStream_t s) {
             case 2: launch_tile<WF, EPI, 2, 4, 2, 1>(a, grid, s); break;
             case 3: launch_tile<WF, EPI, 4, 2, 1, 2>(a, grid, s); break;
             case 5: launch_tile<WF, EPI, 4, 2, 1, 1>(a, grid, s); break;
+            case 9: launch_tile<WF, EPI, 2, 2, 1, 1>(a, grid, s); break;
             default: launch_tile<WF, EPI, 4, 2, 2, 1>(a, grid, s); break;
         }
     } else {
@@ -1417,6 +1418,7 @@ void launch_tiles(int c, const kargs & a, hipStream_t s) {
             case 3: launch_tile<WF, EPI, 4, 2, 1, 2>(a, grid, s); break;
             case 4: launch_tile<WF, EPI, 2, 4, 1, 1>(a, grid, s); break;
             case 5: launch_tile<WF, EPI, 4, 2, 1, 1>(a, grid, s); break;
+            case 9: launch_tile<WF, EPI, 2, 2, 1, 1>(a, grid, s); break;
             default: launch_tile<WF, EPI, 4, 2, 2, 1>(a, grid, s); break;
         }
     }
