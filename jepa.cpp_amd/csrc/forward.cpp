@@ -25,12 +25,13 @@
 #define HIP_OK(expr) \
     do { hipError_t e_ = (expr); if (e_ != hipSuccess) { jepa_log("jepa: %s failed: %s\n", #expr, hipGetErrorString(e_)); return false; } } while (0)
 
-jepa_context::jepa_context() = default;
+jepa_context::jepa_context() : staging(new host_staging()) {}
 
 jepa_context::~jepa_context() {
     std::lock_guard<std::recursive_mutex> lk(jepa_hip_mutex());
     hipSetDevice(device);
     ws.reset();
+    staging.reset();
     if (io_in) hipFree(io_in);
     if (io_out) hipFree(io_out);
     if (ev0) hipEventDestroy(ev0);
@@ -534,10 +535,9 @@ int64_t encode_host(jepa_context * ctx, const jepa_input * in, float * out_host,
     lk.unlock();
     float * din = (float *) ctx->io_in, * dout = (float *) ctx->io_out;
     int64_t r = -1;
-    if (hipMemcpyAsync(din, in->data, n_in * 4, hipMemcpyHostToDevice, ctx->stream) == hipSuccess) {
+    if (ctx->staging->upload(din, in->data, n_in * 4, ctx->stream)) {
         r = encode_device(ctx, din, in->n_batch, in->n_chans, in->n_frames, in->height, in->width, dout, (int64_t) n_out, nullptr, 0);
-        if (r > 0 && (hipMemcpyAsync(out_host, dout, n_out * 4, hipMemcpyDeviceToHost, ctx->stream) != hipSuccess ||
-                      hipStreamSynchronize(ctx->stream) != hipSuccess)) {
+        if (r > 0 && !ctx->staging->download(out_host, dout, n_out * 4, ctx->stream)) {
             jepa_log("jepa: output download failed\n");
             r = -1;
         }

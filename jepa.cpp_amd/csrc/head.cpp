@@ -168,7 +168,7 @@ extern "C" int jepa_head_ex(jepa_context * ctx, const jepa_output * enc, jepa_ou
     }
     if (!head_check_rows(m, N) || hipSetDevice(ctx->device) != hipSuccess || !ensure_head_workspace(ctx, N)) return -1;
     fwd_workspace & w = *ctx->hws;
-    if (hipMemcpyAsync(w.x, enc->data, (size_t) N * D * 4, hipMemcpyHostToDevice, ctx->stream) != hipSuccess) {
+    if (!ctx->staging->upload(w.x, enc->data, (size_t) N * D * 4, ctx->stream)) {
         jepa_log("jepa: input upload failed\n");
         return -1;
     }

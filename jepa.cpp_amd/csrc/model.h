@@ -7,6 +7,7 @@
 #include "../../include/jepa.h"
 #include "common.h"
 #include "gguf.h"
+#include "staging.h"
 
 #include <hip/hip_runtime.h>
 
@@ -200,6 +201,7 @@ struct jepa_context {
     std::unique_ptr<fwd_workspace> ws;
     std::unique_ptr<fwd_workspace> hws;   // jepa_head's buffers, made for the last token count
     std::unique_ptr<fwd_workspace> pws;   // jepa_predict's buffers, made for the last context + target count
+    std::unique_ptr<host_staging> staging;   // pinned memory of the host-buffer calls
     void * io_in = nullptr, * io_out = nullptr;   // device copies of jepa_encode's host input / output
     size_t io_in_cap = 0, io_out_cap = 0;
     // per-kernel timing (jepa_amd_context_set_kernel_timing)

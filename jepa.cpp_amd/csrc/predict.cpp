@@ -102,6 +102,26 @@ bool ensure_pred_workspace(jepa_context * ctx, int n_ctx, int n_tgt) {
     return true;
 }
 
+// the RoPE tables of the tokens ids into w.rope_c / w.rope_s
+bool upload_rope(jepa_context * ctx, const rope3d_params & rp, const int32_t * ids, int64_t N) {
+    fwd_workspace & w = *ctx->pws;
+    std::vector<float> c, sn;
+    rope3d_axis_tables(rp, c, sn);
+    const size_t nb = (size_t) N * 4, tb = c.size() * 4;
+    if (w.rope_src_cap < nb + 2 * tb) {   // (the temporal rows grow with the largest id)
+        std::lock_guard<std::recursive_mutex> lk(jepa_hip_mutex());
+        const size_t cap = 2 * (nb + 2 * tb);
+        if (!ws_alloc(w, &w.rope_src, cap)) { w.rope_src_cap = 0; return false; }
+        w.rope_src_cap = cap;
+    }
+    char * dev = (char *) w.rope_src;
+    if (!ctx->staging->upload(dev, ids, nb, ctx->stream) || !ctx->staging->upload(dev + nb, c.data(), tb, ctx->stream) ||
+        !ctx->staging->upload(dev + nb + tb, sn.data(), tb, ctx->stream)) return false;
+    launch_rope_rows((const int32_t *) dev, (const float *) (dev + nb), (const float *) (dev + nb + tb), N, rp.head_dim,
+                     rope3d_axis_dim(rp.head_dim), rp.grid_t, rp.grid_h, rp.grid_w, w.rope_c, w.rope_s, ctx->stream);
+    return true;
+}
+
 // the predictor on the context rows already in w.pin; target rows into w.pout
 int pred_run(jepa_context * ctx, const int32_t * ids, int n_ctx, int n_tgt, int mask_index, int modality) {
     const jepa_model * m = ctx->model;
@@ -128,12 +148,8 @@ int pred_run(jepa_context * ctx, const int32_t * ids, int n_ctx, int n_tgt, int 
             return -1;
         }
     }
-    std::vector<float> c, sn;
-    rope3d_tables(rp, ids, N, c, sn, true);
     ktimer kt{ctx};
     hipEventRecord(ctx->ev0, s);
-    bool ok = hipMemcpyAsync(w.rope_c, c.data(), c.size() * 4, hipMemcpyHostToDevice, s) == hipSuccess &&
-              hipMemcpyAsync(w.rope_s, sn.data(), sn.size() * 4, hipMemcpyHostToDevice, s) == hipSuccess;
     // 1. context rows -> predictor width (+ modality vector)
     if (n_ctx > 0) {
         const dev_linear & last = pr.embed0.w ? pr.embed2 : pr.embed;
@@ -159,6 +175,10 @@ int pred_run(jepa_context * ctx, const int32_t * ids, int n_ctx, int n_tgt, int 
         kt.run("cls", [&] { launch_cls_rows(w.x + (int64_t) n_ctx * Dp, pr.mask_tokens + idx * Dp, mod, n_tgt, 1, Dp, s); });
     }
     // 3. blocks with 3-D RoPE from the ids
+    if (!upload_rope(ctx, rp, ids, N)) {
+        jepa_log("jepa: jepa_predict: RoPE table upload failed\n");
+        return -1;
+    }
     for (const dev_layer & L : pr.blocks) enqueue_block(b, L, w, 1, N, w.rope_c, w.rope_s, 0, 0, s, kt);
     // 4. final norm of the target rows, projection
     w.actA.fmt = pr.proj.act();
@@ -172,7 +192,7 @@ int pred_run(jepa_context * ctx, const int32_t * ids, int n_ctx, int n_tgt, int 
     }
     hipEventRecord(ctx->ev1, s);
     const hipError_t err = hipStreamSynchronize(s);
-    if (!ok || err != hipSuccess) {
+    if (err != hipSuccess) {
         jepa_log("jepa: jepa_predict: device execution failed: %s\n", hipGetErrorString(err));
         return -1;
     }
@@ -256,10 +276,15 @@ extern "C" int jepa_predict_mod(jepa_context * ctx, const jepa_output * enc, con
     fwd_workspace & w = *ctx->pws;
     // gather the context rows (src/predictor.cpp:187-191), one upload
     if (n_context > 0) {
-        std::vector<float> rows((size_t) n_context * De);
-        for (int i = 0; i < n_context; i++) memcpy(rows.data() + (size_t) i * De, enc->data + (size_t) ids[(size_t) i] * De, (size_t) De * 4);
-        if (hipMemcpyAsync(w.pin, rows.data(), rows.size() * 4, hipMemcpyHostToDevice, ctx->stream) != hipSuccess ||
-            hipStreamSynchronize(ctx->stream) != hipSuccess) {
+        const size_t row = (size_t) De * 4;
+        auto gather = [&](void * p, size_t at, size_t n) {
+            for (size_t done = 0; done < n;) {
+                const size_t i = (at + done) / row, in = (at + done) % row, k = std::min(row - in, n - done);
+                memcpy((char *) p + done, (const char *) (enc->data + (size_t) ids[i] * De) + in, k);
+                done += k;
+            }
+        };
+        if (!ctx->staging->upload(w.pin, (size_t) n_context * row, ctx->stream, gather)) {
             jepa_log("jepa: input upload failed\n");
             return -1;
         }
@@ -268,8 +293,7 @@ extern "C" int jepa_predict_mod(jepa_context * ctx, const jepa_output * enc, con
     if (od < 0) return -1;
     float * data = (float *) malloc((size_t) n_target * od * 4);
     if (!data) return -1;
-    if (hipMemcpyAsync(data, w.pout, (size_t) n_target * od * 4, hipMemcpyDeviceToHost, ctx->stream) != hipSuccess ||
-        hipStreamSynchronize(ctx->stream) != hipSuccess) {
+    if (!ctx->staging->download(data, w.pout, (size_t) n_target * od * 4, ctx->stream)) {
         jepa_log("jepa: output download failed\n");
         free(data);
         return -1;

@@ -19,30 +19,35 @@ float axis_pos(const rope3d_params & p, int axis, int i) {
 
 }  // namespace
 
+void rope3d_axis_tables(const rope3d_params & p, std::vector<float> & c, std::vector<float> & s) {
+    const int d = rope3d_axis_dim(p.head_dim), half = d / 2;
+    const int dims[3] = {p.grid_t, p.grid_h, p.grid_w};
+    c.resize((size_t) (p.grid_t + p.grid_h + p.grid_w) * d);
+    s.resize(c.size());
+    std::vector<float> omega((size_t) half);
+    for (int k = 0; k < half; k++) omega[(size_t) k] = 1.0f / powf(p.theta, (float) k / (float) half);
+    size_t at = 0;
+    for (int a = 0; a < 3; a++)
+        for (int i = 0; i < dims[a]; i++) {
+            const float pos = axis_pos(p, a, i);
+            for (int j = 0; j < d; j++, at++) {
+                const int k = p.variant == 0 ? (j % half) : (j / 2);
+                const float ang = pos * omega[(size_t) k];
+                c[at] = cosf(ang);
+                s[at] = sinf(ang);
+            }
+        }
+}
+
 void rope3d_tables(const rope3d_params & p, const int32_t * ids, int64_t n_rows, std::vector<float> & c,
                    std::vector<float> & s, bool signed_sin) {
-    const int D = p.head_dim, d = rope3d_axis_dim(D), half = d / 2;
+    const int D = p.head_dim, d = rope3d_axis_dim(D);
     c.assign((size_t) n_rows * D, 1.0f);
     s.assign((size_t) n_rows * D, 0.0f);
     if (d == 0) return;
-    std::vector<float> omega((size_t) half);
-    for (int k = 0; k < half; k++) omega[(size_t) k] = 1.0f / powf(p.theta, (float) k / (float) half);
-    const int dims[3] = {p.grid_t, p.grid_h, p.grid_w};
-    // per-axis rows, cached by grid coordinate
-    std::vector<float> ac[3], as[3];
-    for (int a = 0; a < 3; a++) {
-        ac[a].resize((size_t) dims[a] * d);
-        as[a].resize((size_t) dims[a] * d);
-        for (int i = 0; i < dims[a]; i++) {
-            const float pos = axis_pos(p, a, i);
-            for (int j = 0; j < d; j++) {
-                const int k = p.variant == 0 ? (j % half) : (j / 2);
-                const float ang = pos * omega[(size_t) k];
-                ac[a][(size_t) i * d + j] = cosf(ang);
-                as[a][(size_t) i * d + j] = sinf(ang);
-            }
-        }
-    }
+    std::vector<float> ac, as;
+    rope3d_axis_tables(p, ac, as);
+    const int first[3] = {0, p.grid_t, p.grid_t + p.grid_h};   // axis a's first row
     const int64_t per_frame = (int64_t) p.grid_h * p.grid_w;
     for (int64_t r = 0; r < n_rows; r++) {
         const int64_t id = ids ? ids[r] : r;
@@ -51,8 +56,8 @@ void rope3d_tables(const rope3d_params & p, const int32_t * ids, int64_t n_rows,
         float * sr = &s[(size_t) r * D];
         for (int a = 0; a < 3; a++)
             for (int j = 0; j < d; j++) {
-                cr[a * d + j] = ac[a][(size_t) idx[a] * d + j];
-                sr[a * d + j] = as[a][(size_t) idx[a] * d + j];
+                cr[a * d + j] = ac[(size_t) (first[a] + idx[a]) * d + j];
+                sr[a * d + j] = as[(size_t) (first[a] + idx[a]) * d + j];
             }
         if (signed_sin)
             for (int j = 0; j < D; j += 2) sr[j] = -sr[j];

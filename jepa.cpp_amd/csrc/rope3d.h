@@ -20,6 +20,8 @@ struct rope3d_params {
 };
 
 int rope3d_axis_dim(int head_dim);
+// the rows of each axis, [dims[axis]][axis_dim] cosines and (unsigned) sines, t then h then w
+void rope3d_axis_tables(const rope3d_params & p, std::vector<float> & cos_out, std::vector<float> & sin_out);
 // [n_rows, head_dim] tables; ids == nullptr means every token of the grid in T-major order
 void rope3d_tables(const rope3d_params & p, const int32_t * ids, int64_t n_rows, std::vector<float> & cos_out,
                    std::vector<float> & sin_out, bool signed_sin = true);
