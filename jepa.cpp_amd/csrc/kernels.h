@@ -106,9 +106,11 @@ bool launch_pool_attention(const float * q, const float * K, const float * V, in
 void launch_patchify(const float * in, void * rows, bool half_out, int64_t n_items, int C, int T, int H, int W,
                      int P, int tub, bool video, hipStream_t s);
 
-// prefix (CLS) rows: x[it*R + 0][n] = cls[n] (+ pos[n])
+// RoPE tables [n_rows][hd] (signed sine) of the tokens ids from the rows of each axis (rope3d_axis_tables, d wide)
 void launch_rope_rows(const int32_t * ids, const float * ac, const float * as, int64_t n_rows, int hd, int d, int gt, int gh, int gw,
                       float * c, float * s, hipStream_t st);
+
+// prefix (CLS) rows: x[it*R + 0][n] = cls[n] (+ pos[n])
 void launch_cls_rows(float * x, const float * cls, const float * pos, int64_t n_items, int64_t R, int64_t D, hipStream_t s);
 // rows 0 .. (cls ? 1 : 0) + n_reg - 1 of every item of R rows: CLS, then the register rows [n_reg][D],
 // each plus its row of pos when pos is not null

@@ -375,6 +375,20 @@ void launch_prefix_rows(float * x, const float * cls, const float * reg, int n_r
     if (np > 0) k_prefix_rows<<<nblk(n_items * np * D, 256), 256, 0, s>>>(x, cls, reg, n_reg, pos, n_items, R, D);
 }
 
+__global__ void k_copy_bytes(const uint32_t * __restrict__ src, uint32_t * __restrict__ dst, int64_t n, bool wide) {
+    const int64_t i0 = (int64_t) blockIdx.x * blockDim.x + threadIdx.x, step = (int64_t) gridDim.x * blockDim.x;
+    const int64_t n4 = wide ? n / 4 : 0;
+    for (int64_t i = i0; i < n4; i += step) ((uint4 *) dst)[i] = ((const uint4 *) src)[i];
+    for (int64_t i = 4 * n4 + i0; i < n; i += step) dst[i] = src[i];
+}
+
+void launch_copy_bytes(const void * src, void * dst, size_t n, hipStream_t s) {
+    const bool wide = (((uintptr_t) src | (uintptr_t) dst) & 15) == 0;
+    const size_t items = (n / 4 + 3) / 4;
+    if (n >= 4) k_copy_bytes<<<(unsigned) std::min<size_t>(512, (items + 255) / 256), 256, 0, s>>>((const uint32_t *) src, (uint32_t *) dst,
+                                                                                                 (int64_t) (n / 4), wide);
+}
+
 // [n_rows][hd] RoPE tables (signed sine) of the tokens ids, from the rows of each axis (rope3d_axis_tables: the
 // host's cosf and sinf; this only places them). A predictor call of 2048 tokens x 32 sends 11 KB instead of
 // 512 KB, and the host no longer writes the tables (~100 us) before the first launch.
