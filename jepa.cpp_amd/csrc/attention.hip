@@ -429,32 +429,70 @@ __global__ __launch_bounds__(64 * KS * 4 / QT, 1) void k_attn_hd64(const _Float1
 
 // Head widths other than 32 and 64 (80 for I-JEPA ViT-H/14): heads stored HDS = 32 * NDT wide with
 // zero padding past hd (Q, K [head][R_pad][HDS], V^T [head][HDS][R_pad] in the PV order of the 16-token
-// groups, as the QKV epilogue writes them). One workgroup = 4 waves = 128 queries of one head, each wave
-// 32 queries over every key; K and V^T operands are read straight from global memory (L2), which suits
-// the short sequences these models run (256 tokens at 224^2). The arithmetic per 32-key block is the
-// fast kernel's: S^T = K . Q^T over NKK = ceil(hd / 16) dim steps (the padded dims are zero), the lazy
-// online softmax in the exp2 form, O^T += V^T . P^T over NDT 32-dim row blocks. f32 output only: q8_0
-// blocks of 32 dims would span heads.
-template <int NKK, int NDT>
+// groups, as the QKV epilogue writes them). The arithmetic per 32-key block is the fast kernel's:
+// S^T = K . Q^T over NKK = ceil(hd / 16) dim steps (the padded dims are zero), the lazy online softmax
+// in the exp2 form, O^T += V^T . P^T over NDT 32-dim row blocks. Output f32, or the same rounded to
+// f16 (q8_0 blocks of 32 dims would span heads).
+// One workgroup = 4 waves = 64 queries of one head: two query tiles, and of each 64-key stage one wave of a
+// tile takes the first 32 keys and the other the second; the two meet in LDS at the end, first half
+// first. K and V^T stages are copied HBM -> LDS whole lines at a time, two in flight beyond the one
+// computed. Operands read straight from global memory (32 rows per load instruction, each K / V^T row by
+// four waves) kept the address unit busy instead: 256 keys x 64 heads of 80 took 18.5 us with f32
+// rows and a conversion kernel of 5.5 us behind them; now 7.6 us in f16 (128 queries per workgroup also
+// left half of the CUs without work there).
+template <int NKK, int NDT, bool F16>
 __global__ __launch_bounds__(256) void k_attn_any(const _Float16 * __restrict__ Q, const _Float16 * __restrict__ Kp,
-                                                  const _Float16 * __restrict__ Vt, float * __restrict__ O, int n_head,
+                                                  const _Float16 * __restrict__ Vt, void * __restrict__ O, int n_head,
                                                   int hd, int64_t R, int64_t R_pad, float c, int np, int tpf) {
-    constexpr int HDS = 32 * NDT;
-    static_assert(NKK * 16 <= HDS, "dim steps inside the stored width");
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    constexpr int HDS = 32 * NDT, KROW = 2 * HDS, CH = 4 * NDT;   // bytes and 16-byte chunks of a K row
+    constexpr int VOFF = KT * KROW, ANY_STAGE = 2 * VOFF, NS = 3; // a stage: K rows, then V^T rows of 128 B
+    // K rows start at 1, 2 or 4 different chunks modulo 16 (CH r); chunk c of row r sits in slot c with
+    // its low bits xored with r / P, so that the 16 rows one ds_read_b128 pass serves hit 16 bank groups
+    constexpr int P = NDT == 2 ? 2 : NDT == 3 ? 4 : 1, G = 16 / P;
+    static_assert(NKK * 16 <= HDS && NDT >= 2 && NDT <= 4, "dim steps inside the stored width");
+    __shared__ __attribute__((aligned(16))) unsigned char smem[NS * ANY_STAGE];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l32 = lane & 31, g = lane >> 5;
-    const int64_t head = blockIdx.y;
+    const int qt = wave & 1, ks = wave >> 1;
+    // a head's query blocks on one XCD (as in k_attn_hd64)
+    const uint32_t gx = gridDim.x, total = gridDim.x * gridDim.y, lin = blockIdx.x + gx * blockIdx.y;
+    const uint32_t rl = total % 8 == 0 ? (lin % 8) * (total / 8) + lin / 8 : lin;
+    const uint32_t qblk = rl % gx;
+    const int64_t head = rl / gx;
     const int64_t item = head / n_head;
     const int h = (int) (head - item * n_head);
-    const int64_t q0 = (int64_t) blockIdx.x * 128 + 32 * wave;
-    if (q0 >= R) return;                                  // whole wave past the last query
+    const int64_t q0 = (int64_t) qblk * 64 + 32 * qt;
     const _Float16 * Qh = Q + head * R_pad * HDS;
-    const _Float16 * Kh = Kp + head * R_pad * HDS;
-    const _Float16 * Vh = Vt + head * HDS * R_pad;
+    const brsrc rK = make_brsrc(Kp + head * R_pad * HDS, R_pad * KROW);
+    const brsrc rV = make_brsrc(Vt + head * HDS * R_pad, R_pad * KROW);
 
+    const int qa = (int) qblk * 64, qz = min((int) R, qa + 64) - 1;
+    const int klo_wg = key_range(qa, (int) R, np, tpf).x;
+    const int khi_wg = qa < np ? (int) R : key_range(qz, (int) R, np, tpf).y;
+    const int t0 = klo_wg / KT, nt = (khi_wg + KT - 1) / KT - t0;
+    // copy i of this wave fills 64 slots of the stage: the first NDT copies K, the others V^T
+    uint32_t src[2 * NDT];
+#pragma unroll
+    for (int i = 0; i < NDT; i++) {
+        const int x = 64 * (4 * i + wave) + lane, r = x / CH, t = x - r * CH;
+        src[i] = (uint32_t) r * KROW + 16 * ((t & ~(G - 1)) | ((t ^ (r / P)) & (G - 1)));
+        const int d = x >> 3;
+        src[NDT + i] = (uint32_t) d * (uint32_t) R_pad * 2 + 16 * lds_slot(d, x & 7);
+    }
+    auto issue = [&](int s) {
+        if (s >= nt) return;
+        unsigned char * base = smem + (s % NS) * ANY_STAGE;
+        const uint32_t key0 = (uint32_t) (t0 + s) * KT;
+#pragma unroll
+        for (int i = 0; i < NDT; i++) dma_to_lds<16>(rK, src[i], key0 * KROW, base + 1024 * (4 * i + wave));
+#pragma unroll
+        for (int i = 0; i < NDT; i++) dma_to_lds<16>(rV, src[NDT + i], key0 * 2, base + VOFF + 1024 * (4 * i + wave));
+    };
     h8 qv[NKK];
 #pragma unroll
     for (int kk = 0; kk < NKK; kk++) qv[kk] = *(const h8 *) (Qh + (q0 + l32) * HDS + 16 * kk + 8 * g);
+    issue(0);
+    issue(1);
 
     const f16v zero = {0};
     f16v acc[NDT];
@@ -463,19 +501,36 @@ __global__ __launch_bounds__(256) void k_attn_any(const _Float16 * __restrict__ 
     // the running maximum in the exp2 domain, as in k_attn_hd64: mcs, its negation nm, threshold thr
     float mcs = -INFINITY, nm = 0.0f, thr = -INFINITY, l_run = 0.0f;
     const int2 kr = key_range((int) q0 + l32, (int) R, np, tpf);
-    const int qw = (int) q0;
-    const int lo_min = key_range(qw, (int) R, np, tpf).x;
-    const int hi_max = qw < np ? (int) R : key_range(min(qw + 31, (int) R - 1), (int) R, np, tpf).y;
+    const int qw = (int) q0, qp = max(qw, np);
+    const int lo_max = key_range(qw + 31, (int) R, np, tpf).x;
+    const int hi_min = qp <= qw + 31 ? key_range(qp, (int) R, np, tpf).y : (int) R;
     const h2 one2 = {(_Float16) 1.0f, (_Float16) 1.0f};
-    for (int kb0 = (lo_min / 32) * 32; kb0 < hi_max; kb0 += 32) {
+    for (int s = 0; s < nt; s++) {
+        // stage s has landed (at most the copies of stage s + 1 outstanding) and every wave is past stage
+        // s - 1, whose buffer stage s + 2 refills
+        if (s + 1 < nt) tile_barrier<2 * NDT>();
+        else tile_barrier<0>();
+        issue(s + 2);
+        const unsigned char * sK = smem + (s % NS) * ANY_STAGE, * sV = sK + VOFF;
+        const int kb0 = (t0 + s) * KT + 32 * ks, row = 32 * ks + l32;
         f16v S = zero;
 #pragma unroll
-        for (int kk = 0; kk < NKK; kk++) S = MFMA16(*(const h8 *) (Kh + (int64_t) (kb0 + l32) * HDS + 16 * kk + 8 * g), qv[kk], S);
-        const int key0 = kb0 + 4 * g;
+        for (int kk = 0; kk < NKK; kk++) {
+            const int ch = 2 * kk + g, slot = (ch & ~(G - 1)) | ((ch ^ (row / P)) & (G - 1));
+            S = MFMA16(*(const h8 *) (sK + row * KROW + 16 * slot), qv[kk], S);
+        }
+        h8 vc[2][NDT];
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const int key = key0 + 8 * (r >> 2) + (r & 3);
-            if (key < kr.x || key >= kr.y) S[r] = -INFINITY;
+        for (int kk2 = 0; kk2 < 2; kk2++)
+#pragma unroll
+            for (int dt = 0; dt < NDT; dt++) vc[kk2][dt] = lds_chunk(sV, 32 * dt + l32, 4 * ks + 2 * kk2 + g);
+        if (kb0 < lo_max || kb0 + 32 > hi_min) {
+            const int key0 = kb0 + 4 * g;
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int key = key0 + 8 * (r >> 2) + (r & 3);
+                if (key < kr.x || key >= kr.y) S[r] = -INFINITY;
+            }
         }
 #pragma unroll
         for (int r = 0; r < 16; r++) S[r] = fmaf(S[r], c, nm);
@@ -483,19 +538,22 @@ __global__ __launch_bounds__(256) void k_attn_any(const _Float16 * __restrict__ 
 #pragma unroll
         for (int r = 3; r < 15; r += 2) tl = fmaxf(fmaxf(tl, S[r]), S[r + 1]);
         tl = halves_max_nonan(fmaxf(tl, S[15]));
-        if (tl > thr) {
+        const bool move = tl > thr;
+        if (__builtin_amdgcn_ballot_w64(move) != 0) {
+            asm volatile("");
             const bool first = mcs == -INFINITY;
-            const float alpha = first ? 0.0f : fast_exp2(-tl);
+            const float sh = move ? tl : 0.0f;
+            const float alpha = first ? 0.0f : fast_exp2(-sh);
             l_run *= alpha;
 #pragma unroll
             for (int dt = 0; dt < NDT; dt++)
 #pragma unroll
                 for (int r = 0; r < 16; r++) acc[dt][r] *= alpha;
 #pragma unroll
-            for (int r = 0; r < 16; r++) S[r] = __fsub_rn(S[r], tl);
-            mcs = first ? tl : mcs + tl;
-            nm = -mcs;
-            thr = LAZY;
+            for (int r = 0; r < 16; r++) S[r] = __fsub_rn(S[r], sh);
+            mcs = move ? (first ? tl : mcs + tl) : mcs;
+            nm = mcs == -INFINITY ? 0.0f : -mcs;
+            thr = mcs == -INFINITY ? -INFINITY : LAZY;
         }
         float lsum = 0.0f;
 #pragma unroll
@@ -505,25 +563,42 @@ __global__ __launch_bounds__(256) void k_attn_any(const _Float16 * __restrict__ 
             for (int e = 0; e < 8; e++) pb[e] = (_Float16) fast_exp2(S[8 * kk2 + e]);
 #pragma unroll
             for (int e = 0; e < 4; e++) lsum = __builtin_amdgcn_fdot2(h2{pb[2 * e], pb[2 * e + 1]}, one2, lsum, false);
-            // V^T row d, keys kb0 + 16 kk2 + 8 g .. + 8 in the order of the S lanes (see the header)
 #pragma unroll
-            for (int dt = 0; dt < NDT; dt++)
-                acc[dt] = MFMA16(*(const h8 *) (Vh + (int64_t) (32 * dt + l32) * R_pad + kb0 + 16 * kk2 + 8 * g), pb, acc[dt]);
+            for (int dt = 0; dt < NDT; dt++) acc[dt] = MFMA16(vc[kk2][dt], pb, acc[dt]);
         }
         l_run += halves_sum(lsum);
     }
+
+    // the second halves publish (m, l, acc) through LDS, the first add them (as in k_attn_hd64)
+    __syncthreads();
+    float * xs = (float *) smem + (size_t) qt * (2 + 16 * NDT) * 64 + lane;
+    if (ks > 0) {
+        xs[0] = mcs; xs[64] = l_run;
+#pragma unroll
+        for (int dt = 0; dt < NDT; dt++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) xs[(2 + 16 * dt + r) * 64] = acc[dt][r];
+    }
+    __syncthreads();
     const int64_t q = q0 + l32;
-    if (q >= R) return;
-    const float inv = l_run > 0.0f ? 1.0f / l_run : 0.0f;
-    float * orow = O + (item * R + q) * ((int64_t) n_head * hd) + (int64_t) h * hd;
+    if (ks > 0 || q >= R) return;
+    const float m1 = xs[0], m = fmaxf(mcs, m1);
+    const float a0 = mcs == -INFINITY ? 0.0f : fast_exp2(mcs - m), a1 = m1 == -INFINITY ? 0.0f : fast_exp2(m1 - m);
+    const float l = fmaf(xs[64], a1, l_run * a0), inv = l > 0.0f ? 1.0f / l : 0.0f;
+    const int64_t at = (item * R + q) * ((int64_t) n_head * hd) + (int64_t) h * hd;
 #pragma unroll
     for (int dt = 0; dt < NDT; dt++)
 #pragma unroll
         for (int qq = 0; qq < 4; qq++) {
             const int d = 32 * dt + 8 * qq + 4 * g;
-            if (d < hd)   // hd is a multiple of 16: a group of four is inside or outside as a whole
-                *(float4 *) (orow + d) = make_float4(acc[dt][4 * qq] * inv, acc[dt][4 * qq + 1] * inv, acc[dt][4 * qq + 2] * inv,
-                                                     acc[dt][4 * qq + 3] * inv);
+            float o[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++) o[e] = fmaf(xs[(2 + 16 * dt + 4 * qq + e) * 64], a1, acc[dt][4 * qq + e] * a0) * inv;
+            if (d < hd) {   // hd is a multiple of 16: a group of four is inside or outside as a whole
+                typedef _Float16 h4o __attribute__((ext_vector_type(4)));
+                if constexpr (F16) *(h4o *) ((_Float16 *) O + at + d) = h4o{(_Float16) o[0], (_Float16) o[1], (_Float16) o[2], (_Float16) o[3]};
+                else *(float4 *) ((float *) O + at + d) = make_float4(o[0], o[1], o[2], o[3]);
+            }
         }
 }
 
@@ -545,20 +620,26 @@ void launch_attention(const void * q, const void * k, const void * vt, const act
                       int n_head, int hd, int64_t R, int64_t R_pad, float scale, int n_prefix, int64_t tokens_per_slot,
                       hipStream_t s) {
     // hd: 64, or 32 (stored 64 wide), or a multiple of 16 up to 128 stored attention_stored_width(hd)
-    // wide (f32 output; checked by the callers)
+    // wide (f32 or f16 output; checked by the callers)
     const float c = scale * 1.4426950408889634f;   // exp(x*scale) = exp2(x*scale*log2(e))
     const int tpf = (int) tokens_per_slot;
     dim3 grid((unsigned) ((R + QB - 1) / QB), (unsigned) (n_items * n_head));
     const _Float16 * Q = (const _Float16 *) q, * K = (const _Float16 *) k, * V = (const _Float16 *) vt;
     if (hd != 32 && hd != 64) {
-        float * o = (float *) out.q;
+        const dim3 ag((unsigned) ((R + 63) / 64), (unsigned) (n_items * n_head));
+        auto any = [&](auto nkk, auto ndt) {
+            constexpr int NKK = decltype(nkk)::value, NDT = decltype(ndt)::value;
+            if (out.fmt == A_F16) k_attn_any<NKK, NDT, true><<<ag, 256, 0, s>>>(Q, K, V, out.q, n_head, hd, R, R_pad, c, n_prefix, tpf);
+            else k_attn_any<NKK, NDT, false><<<ag, 256, 0, s>>>(Q, K, V, out.q, n_head, hd, R, R_pad, c, n_prefix, tpf);
+        };
+        using std::integral_constant;
         switch ((hd + 15) / 16) {
-            case 1: k_attn_any<1, 2><<<grid, 256, 0, s>>>(Q, K, V, o, n_head, hd, R, R_pad, c, n_prefix, tpf); break;
-            case 3: k_attn_any<3, 2><<<grid, 256, 0, s>>>(Q, K, V, o, n_head, hd, R, R_pad, c, n_prefix, tpf); break;
-            case 5: k_attn_any<5, 3><<<grid, 256, 0, s>>>(Q, K, V, o, n_head, hd, R, R_pad, c, n_prefix, tpf); break;
-            case 6: k_attn_any<6, 3><<<grid, 256, 0, s>>>(Q, K, V, o, n_head, hd, R, R_pad, c, n_prefix, tpf); break;
-            case 7: k_attn_any<7, 4><<<grid, 256, 0, s>>>(Q, K, V, o, n_head, hd, R, R_pad, c, n_prefix, tpf); break;
-            case 8: k_attn_any<8, 4><<<grid, 256, 0, s>>>(Q, K, V, o, n_head, hd, R, R_pad, c, n_prefix, tpf); break;
+            case 1: any(integral_constant<int, 1>{}, integral_constant<int, 2>{}); break;
+            case 3: any(integral_constant<int, 3>{}, integral_constant<int, 2>{}); break;
+            case 5: any(integral_constant<int, 5>{}, integral_constant<int, 3>{}); break;
+            case 6: any(integral_constant<int, 6>{}, integral_constant<int, 3>{}); break;
+            case 7: any(integral_constant<int, 7>{}, integral_constant<int, 4>{}); break;
+            case 8: any(integral_constant<int, 8>{}, integral_constant<int, 4>{}); break;
             default: break;
         }
         return;

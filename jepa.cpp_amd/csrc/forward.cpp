@@ -197,7 +197,7 @@ void enqueue_block(const blk_shape & b, const dev_layer & L, fwd_workspace & w, 
         }
     }
     w.actA.fmt = L.out.act();
-    if ((w.actA.fmt == A_Q8_0 || w.actA.fmt == A_F16) && (hd == 64 || hd == 32)) {
+    if (w.actA.fmt == A_F16 || (w.actA.fmt == A_Q8_0 && (hd == 64 || hd == 32))) {
         // the attention epilogue writes the out-projection's q8_0 or f16 input directly
         kt.run("attention", [&] {
             launch_attention(w.Q, w.Kt, w.Vt, w.actA, n_items, H, hd, R, w.R_pad, 1.0f / sqrtf((float) hd), n_prefix, slot_rows, s);

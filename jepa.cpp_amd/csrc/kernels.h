@@ -90,7 +90,7 @@ void launch_rownorm_quant(const float * x, int64_t M, int64_t D, const float * w
 int attention_key_splits(int64_t R);
 void launch_attention(const void * q, const void * k, const void * vt, const act_view & out, int64_t n_items, int n_head,
                       int hd, int64_t R, int64_t R_pad, float scale, int n_prefix, int64_t tokens_per_slot, hipStream_t s);
-// Head widths the attention runs: 32, 64, and other multiples of 16 up to 128 (f32 output only); the
+// Head widths the attention runs: 32, 64, and other multiples of 16 up to 128 (f32 or f16 output); the
 // width Q, K and V^T are stored with (64 for hd <= 64, else hd rounded up to 32; the rest zero).
 bool attention_supports(int hd);
 int attention_stored_width(int hd);

@@ -145,9 +145,10 @@ __device__ __forceinline__ int16_t tile_tap(const axis_filter & f, double unit, 
 // they are used), waves take the source rows in turn. Four pixels are twelve bytes, loaded as dwords
 // and realigned; v_perm makes pairs of one channel, v_dot2_i32_i16 sums them with pairs of taps.
 // Vertical pass: a thread takes four columns of one channel and pairs of rows.
-// Sixteen 720 x 1280 frames to 256 x 256 of short edge 292 (sides measured on one card): the two
-// kernels and the five table uploads 61 us of kernels, most of it in three byte loads per tap and
-// 11.8 MB of intermediate written and read back; see the dispatch for this one.
+// Sixteen 720 x 1280 frames to 256 x 256 of short edge 292: 19 us, where the two kernels and the five
+// table uploads took 61 us of kernels, most of it in three byte loads per tap and 11.8 MB of
+// intermediate written and read back (22 MB in and 12.6 MB out would take 4.5 us at the card's copy rate:
+// the taps' VALU work and the latency of each row's loads bound it now).
 template <int NC>
 __global__ __launch_bounds__(256) void k_resize_tile(const uint8_t * __restrict__ src, float * __restrict__ out, int n, int h, int w,
                                                      int crop, int oy, int ox, int tx, int ty, axis_filter fx, axis_filter fy, int xshift,

@@ -636,6 +636,27 @@ def test_attention_block_causal(jlib, oracle, n_items, gt, gh, gw, n_prefix, H):
     np.testing.assert_array_equal(host(oq), want.reshape(host(oq).shape))
 
 
+# the staged kernel of the other widths at the edges of its 64-query blocks and 64-key stages, every stored width,
+# one key to several stages (all three buffers in use), and the block-causal mask over shifted slots
+@pytest.mark.parametrize("hd", [16, 48, 80, 96, 112, 128])
+@pytest.mark.parametrize("n_items,n_tok,n_prefix,slot", [(1, 1, 0, 0), (3, 63, 0, 0), (2, 64, 0, 0), (1, 65, 0, 0), (1, 449, 0, 0), (2, 193, 1, 48)])
+def test_attention_other_widths_stages(jlib, oracle, n_items, n_tok, n_prefix, slot, hd):
+    H = 2
+    rng = np.random.default_rng(n_tok + hd)
+    D = H * hd
+    qkv = (rng.standard_normal((n_items * n_tok, 3 * D)) * 1.5).astype(np.float32)
+    mask = oracle.block_causal_mask((n_tok - n_prefix) // slot, 6, 8, n_prefix).astype(np.float64) if slot else None
+    out = torch.full((n_items * n_tok, D), float("nan"), dtype=torch.float32, device="cuda")
+    dq = dev(qkv)
+    r = jlib.lib().jepa_amd_attention(0, dq.data_ptr(), n_items, n_tok, H, hd, None, None, n_prefix, slot, 0, out.data_ptr())
+    assert r == 0, jlib.error_text()
+    got = host(out).astype(np.float64)
+    ref = _attention_ref(qkv, n_items, n_tok, H, None, mask, hd=hd)
+    # f16 keys, values and weights: 2^-11 each (the bars of the other attention tests)
+    assert np.abs(got - ref).max() / np.abs(ref).max() <= 1e-2
+    assert ((got * ref).sum(1) / (np.linalg.norm(got, axis=1) * np.linalg.norm(ref, axis=1))).min() >= 0.9999
+
+
 @pytest.mark.parametrize("n_items,n_tok,H", [(1, 2048, 4), (2, 197, 6), (1, 65, 2)])
 def test_attention_fused_q8_0_equals_separate_quantizer(jlib, oracle, n_items, n_tok, H):
     """The attention epilogue's q8_0 output is byte-identical to quantizing the f32 attention output
