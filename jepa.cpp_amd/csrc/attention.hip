@@ -432,7 +432,7 @@ __global__ __launch_bounds__(64 * KS * 4 / QT, 1) void k_attn_hd64(const _Float1
 // groups, as the QKV epilogue writes them). The arithmetic per 32-key block is the fast kernel's:
 // S^T = K . Q^T over NKK = ceil(hd / 16) dim steps (the padded dims are zero), the lazy online softmax
 // in the exp2 form, O^T += V^T . P^T over NDT 32-dim row blocks. Output f32, or the same rounded to
-// f16 (q8_0 blocks of 32 dims would span heads).
+// f16; heads of 64 also q8_0 (elsewhere blocks of 32 dims would span heads).
 // One workgroup = 4 waves = 64 queries of one head: two query tiles, and of each 64-key stage one wave of a
 // tile takes the first 32 keys and the other the second; the two meet in LDS at the end, first half
 // first. K and V^T stages are copied HBM -> LDS whole lines at a time, two in flight beyond the one
@@ -440,9 +440,9 @@ __global__ __launch_bounds__(64 * KS * 4 / QT, 1) void k_attn_hd64(const _Float1
 // four waves) kept the address unit busy instead: 256 keys x 64 heads of 80 took 18.5 us with f32
 // rows and a conversion kernel of 5.5 us behind them; now 7.6 us in f16 (128 queries per workgroup also
 // left half of the CUs without work there).
-template <int NKK, int NDT, bool F16>
+template <int NKK, int NDT, int OUT>
 __global__ __launch_bounds__(256) void k_attn_any(const _Float16 * __restrict__ Q, const _Float16 * __restrict__ Kp,
-                                                  const _Float16 * __restrict__ Vt, void * __restrict__ O, int n_head,
+                                                  const _Float16 * __restrict__ Vt, void * __restrict__ O, void * __restrict__ Od, int n_head,
                                                   int hd, int64_t R, int64_t R_pad, float c, int np, int tpf) {
     constexpr int HDS = 32 * NDT, KROW = 2 * HDS, CH = 4 * NDT;   // bytes and 16-byte chunks of a K row
     constexpr int VOFF = KT * KROW, ANY_STAGE = 2 * VOFF, NS = 3; // a stage: K rows, then V^T rows of 128 B
@@ -581,35 +581,64 @@ __global__ __launch_bounds__(256) void k_attn_any(const _Float16 * __restrict__ 
     }
     __syncthreads();
     const int64_t q = q0 + l32;
-    if (ks > 0 || q >= R) return;
+    if (ks > 0) return;
     const float m1 = xs[0], m = fmaxf(mcs, m1);
     const float a0 = mcs == -INFINITY ? 0.0f : fast_exp2(mcs - m), a1 = m1 == -INFINITY ? 0.0f : fast_exp2(m1 - m);
     const float l = fmaf(xs[64], a1, l_run * a0), inv = l > 0.0f ? 1.0f / l : 0.0f;
-    const int64_t at = (item * R + q) * ((int64_t) n_head * hd) + (int64_t) h * hd;
+    const int64_t DD = (int64_t) n_head * hd, at = (item * R + q) * DD + (int64_t) h * hd;
 #pragma unroll
-    for (int dt = 0; dt < NDT; dt++)
+    for (int dt = 0; dt < NDT; dt++) {
+        float o[16];
 #pragma unroll
-        for (int qq = 0; qq < 4; qq++) {
-            const int d = 32 * dt + 8 * qq + 4 * g;
-            float o[4];
+        for (int r = 0; r < 16; r++) o[r] = fmaf(xs[(2 + 16 * dt + r) * 64], a1, acc[dt][r] * a0) * inv;
+        if constexpr (OUT == A_Q8_0) {
+            // heads of 64: a 32-dim row block is one q8_0 block, split over lanes l32 and l32 + 32
+            static_assert(NKK == 2 * NDT, "whole blocks of 32");
+            float am = 0.0f;
 #pragma unroll
-            for (int e = 0; e < 4; e++) o[e] = fmaf(xs[(2 + 16 * dt + 4 * qq + e) * 64], a1, acc[dt][4 * qq + e] * a0) * inv;
-            if (d < hd) {   // hd is a multiple of 16: a group of four is inside or outside as a whole
-                typedef _Float16 h4o __attribute__((ext_vector_type(4)));
-                if constexpr (F16) *(h4o *) ((_Float16 *) O + at + d) = h4o{(_Float16) o[0], (_Float16) o[1], (_Float16) o[2], (_Float16) o[3]};
-                else *(float4 *) ((float *) O + at + d) = make_float4(o[0], o[1], o[2], o[3]);
+            for (int r = 0; r < 16; r++) am = fmaxf(am, fabsf(o[r]));
+            am = halves_max(am);
+            const float id = am != 0.0f ? 127.0f / am : 0.0f;
+            if (q >= R) continue;
+#pragma unroll
+            for (int qq = 0; qq < 4; qq++) {
+                uint32_t w = 0;
+#pragma unroll
+                for (int e = 0; e < 4; e++) w |= q8_byte(o[4 * qq + e], id) << (8 * e);
+                *(uint32_t *) ((int8_t *) O + at + 32 * dt + 8 * qq + 4 * g) = w;
+            }
+            if (g == 0) ((uint16_t *) Od)[(item * R + q) * (DD / 32) + h * NDT + dt] = f2hbits(am / 127.0f);
+        } else {
+#pragma unroll
+            for (int qq = 0; qq < 4; qq++) {
+                const int d = 32 * dt + 8 * qq + 4 * g;
+                if (d < hd && q < R) {   // hd is a multiple of 16: a group of four is inside or outside as a whole
+                    typedef _Float16 h4o __attribute__((ext_vector_type(4)));
+                    const float * v = o + 4 * qq;
+                    if constexpr (OUT == A_F16)
+                        *(h4o *) ((_Float16 *) O + at + d) = h4o{(_Float16) v[0], (_Float16) v[1], (_Float16) v[2], (_Float16) v[3]};
+                    else *(float4 *) ((float *) O + at + d) = make_float4(v[0], v[1], v[2], v[3]);
+                }
             }
         }
+    }
 }
 
 }  // namespace
+
+// Heads of 64 over at most this many keys run k_attn_any: 64 queries per workgroup and two waves per query tile fill
+// more CUs, and a wave's chain over the keys is half as long. us, f16 output, k_attn_hd64 / k_attn_any: 101 keys x 6
+// heads 7.5 / 5.0, 197 x 6 10.1 / 6.0 (one image; 8.0 / 6.9 inside a ViT-S/16 call), 256 x 12 7.2 / 5.7, 256 x 96
+// 7.2 / 7.3. Above, a batch pays for the shorter query blocks (576 x 12 10.9 / 8.0, but 576 x 96 16.9 / 20.0),
+// and the choice must not look at the batch: an item's result does not depend on it.
+constexpr int64_t ATTN_FEW_KEYS = 256;
 
 int attention_stored_width(int hd) { return hd <= 64 ? 64 : (hd + 31) / 32 * 32; }
 
 // Key splits by the key count R only (so an item's result does not depend on the batch). Fewer
 // splits mean fewer waves per workgroup, less LDS (32 KB per split) and no merge, and more workgroups
 // per CU. Measured (us per launch, q8_0 output, splits 1 / 2 / 4): 197 keys x 6 heads 8.1 / 8.0 /
-// 10.4, 576 x 96 17.7 / 18.2 / 24.9, 2048 x 16 34.1 / 27.8 / 27.9, 8192 x 22 461 / 461 / 481.
+// 10.4 (now k_attn_any's), 576 x 96 17.7 / 18.2 / 24.9, 2048 x 16 34.1 / 27.8 / 27.9, 8192 x 22 461 / 461 / 481.
 int attention_key_splits(int64_t R) {
     return R <= 1024 ? 1 : R <= 4096 ? 4 : 2;
 }
@@ -625,17 +654,20 @@ void launch_attention(const void * q, const void * k, const void * vt, const act
     const int tpf = (int) tokens_per_slot;
     dim3 grid((unsigned) ((R + QB - 1) / QB), (unsigned) (n_items * n_head));
     const _Float16 * Q = (const _Float16 *) q, * K = (const _Float16 *) k, * V = (const _Float16 *) vt;
-    if (hd != 32 && hd != 64) {
+    if (hd != 32 && (hd != 64 || R <= ATTN_FEW_KEYS)) {
         const dim3 ag((unsigned) ((R + 63) / 64), (unsigned) (n_items * n_head));
         auto any = [&](auto nkk, auto ndt) {
             constexpr int NKK = decltype(nkk)::value, NDT = decltype(ndt)::value;
-            if (out.fmt == A_F16) k_attn_any<NKK, NDT, true><<<ag, 256, 0, s>>>(Q, K, V, out.q, n_head, hd, R, R_pad, c, n_prefix, tpf);
-            else k_attn_any<NKK, NDT, false><<<ag, 256, 0, s>>>(Q, K, V, out.q, n_head, hd, R, R_pad, c, n_prefix, tpf);
+            if (out.fmt == A_F16) k_attn_any<NKK, NDT, A_F16><<<ag, 256, 0, s>>>(Q, K, V, out.q, nullptr, n_head, hd, R, R_pad, c, n_prefix, tpf);
+            else if (out.fmt == A_F32) k_attn_any<NKK, NDT, A_F32><<<ag, 256, 0, s>>>(Q, K, V, out.q, nullptr, n_head, hd, R, R_pad, c, n_prefix, tpf);
+            else if constexpr (NKK == 4)
+                k_attn_any<4, 2, A_Q8_0><<<ag, 256, 0, s>>>(Q, K, V, out.q, out.d, n_head, hd, R, R_pad, c, n_prefix, tpf);
         };
         using std::integral_constant;
         switch ((hd + 15) / 16) {
             case 1: any(integral_constant<int, 1>{}, integral_constant<int, 2>{}); break;
             case 3: any(integral_constant<int, 3>{}, integral_constant<int, 2>{}); break;
+            case 4: any(integral_constant<int, 4>{}, integral_constant<int, 2>{}); break;
             case 5: any(integral_constant<int, 5>{}, integral_constant<int, 3>{}); break;
             case 6: any(integral_constant<int, 6>{}, integral_constant<int, 3>{}); break;
             case 7: any(integral_constant<int, 7>{}, integral_constant<int, 4>{}); break;
