@@ -1546,6 +1546,8 @@ void launch_gemm(const dev_linear & W, const act_view & X, int64_t M, const gemm
         launch_gemm_f32(W, X, M, a.ep, s);
         return;
     }
+    // one row: not where a test hook asks for a tile or a split
+    if (M == 1 && W.fmt == W_Q32 && g_force_tile.load() < 0 && g_force_split.load() < 1 && launch_gemv_q8(W, X, a.ep, s)) return;
     switch (W.fmt) {
         case W_F16: dispatch_mfma<W_F16>(a, s, sw); break;
         case W_Q32: dispatch_mfma<W_Q32>(a, s, sw); break;

@@ -70,6 +70,8 @@ void launch_gemm(const dev_linear & W, const act_view & X, int64_t M, const gemm
                  const gemm_split_ws * sw = nullptr);
 // the same for f32 weights and activations (launch_gemm's W_F32 case; gemm_f32.hip)
 void launch_gemm_f32(const dev_linear & W, const act_view & X, int64_t M, const gemm_epi & ep, hipStream_t s);
+// the same for one row and q8_0 codes (launch_gemm's M == 1; gemv_q8.hip); false: not this format, shape or epilogue
+bool launch_gemv_q8(const dev_linear & W, const act_view & X, const gemm_epi & ep, hipStream_t s);
 // K halves the int8 / 4-bit GEMM of this weight format and shape runs in (1 or 2); depends on N and K
 // only, so that the summation order of an output never depends on the number of rows (f16 weights:
 // chosen per launch from the tile count, 1 here)

@@ -572,6 +572,35 @@ def test_attention_hd32(jlib, oracle, n_items, n_tok, H, rope):
     np.testing.assert_array_equal(host(oq), want.reshape(host(oq).shape))
 
 
+# one row of q8_0 codes has a kernel of its own (block sums by v_dot4, the same fma chain): the same bits as that
+# row among others through the tile kernel; K from two blocks to the largest whose 32 features fit its LDS, and past it
+@pytest.mark.parametrize("N,K", [(128, 64), (384, 320), (1024, 1024), (256, 4096), (128, 5888), (128, 6144)])
+def test_one_row_q8_0_equals_tile_kernel(jlib, N, K):
+    rng = np.random.default_rng(N + K)
+    w = (rng.standard_normal((N, K)) * 0.05).astype(np.float32)
+    w[0, :32] = 0.0
+    x = (rng.standard_normal((3, K)) * 2).astype(np.float32)
+    x[0, 32:64] = 0.0
+    raw, bias = dev(gguf.quantize(gguf.GGML_Q8_0, w).reshape(-1)), dev(rng.standard_normal(N).astype(np.float32))
+    L = jlib.lib()
+
+    def run(rows, gelu):
+        d = dev(x[:rows])
+        n = N // 32 * 34 if gelu else N * 4
+        out = torch.full((rows * n,), 77, dtype=torch.uint8, device="cuda")
+        torch.cuda.synchronize()
+        if gelu:
+            r = L.jepa_amd_matmul_gelu(0, gguf.GGML_Q8_0, raw.data_ptr(), N, K, bias.data_ptr(), d.data_ptr(), rows, gguf.GGML_Q8_0,
+                                       out.data_ptr(), 1, None)
+        else:
+            r = L.jepa_amd_matmul(0, gguf.GGML_Q8_0, raw.data_ptr(), N, K, bias.data_ptr(), d.data_ptr(), rows, out.data_ptr(), 1, None)
+        assert r == 0, jlib.error_text()
+        return host(out)[:n]
+
+    for gelu in (False, True):
+        np.testing.assert_array_equal(run(1, gelu), run(3, gelu))
+
+
 # other head widths (multiples of 16 up to 128, stored rounded up to 32 with zero padding): 80 is I-JEPA
 # ViT-H/14's (16 heads of 80, 256 tokens, RoPE from the reference's hd-80 table layout); 48 and 128 bound
 # the range. Against the double softmax; the q8_0 output is refused (its 32-dim blocks would span heads).
