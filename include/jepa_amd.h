@@ -103,9 +103,10 @@ int jepa_amd_preprocess_frames_device(int device, const jepa_preprocess_params *
  * whose scratch would exceed it (about n_frames * h * crop * 3 bytes plus the tables) is refused
  * with -1 and a message. Work is queued on `stream` (a hipStream_t of `device`; NULL: the null
  * stream) and the call returns without waiting for it; the output is, bit for bit, that of
- * jepa_amd_preprocess_frames_device. Nothing is copied from host memory: the tables reach the
- * device as kernel arguments, so the call can be captured into a HIP graph (make one call on the
- * device before capturing, which looks up the array's address) and the graph replayed on new frames
+ * jepa_amd_preprocess_frames_device. Most calls run a kernel that needs neither tables nor the array;
+ * nothing is copied from host memory in any (tables, where there are some, reach the device as kernel
+ * arguments), so the call can be captured into a HIP graph (make one call on the device before
+ * capturing, which looks up the array's address) and the graph replayed on new frames
  * of the same geometry. Calls on one GPU share the array: calls whose work overlaps on one GPU (on
  * different streams, or graph replays beside eager calls) race, and the caller orders them. */
 int jepa_amd_preprocess_frames_device_noalloc(int device, const jepa_preprocess_params * p, const uint8_t * frames_dev, int n_frames,

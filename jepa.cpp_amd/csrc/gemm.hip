@@ -1311,11 +1311,15 @@ __global__ __launch_bounds__(64 * WN * WM, 1) void k_gemm_mfma(const void * pA, 
 }
 
 struct tile_cfg { int wn, wm, ti, tj; };
-// eight-wave workgroup tiles (BN x BM): 256x128, 192x128, 128x128 (two wave shapes), 64x128, 128x64,
+// Workgroup tiles (BN x BM). The last, 64x64 of four waves (one per SIMD, so less per CU and second than two would
+// do), has the efficiency at which the rule takes it where it means one round of more workgroups and the
+// 128x64 tile would leave CUs idle: us for 128x64 / 64x64, q8_0 576 x 768 x 3072 20.5 / 17.7, 2048 x 384 x 1536
+// 12.4 / 11.0, 1024 x 1024 x 1024 10.3 / 9.1, but 4608 x 768 x 768 14.2 (128x128) / 16.7. Eight-wave tiles: 256x128, 192x128, 128x128 (two wave shapes), 64x128, 128x64,
 // 256x64 (two wave shapes; the second, one weight tile and two token tiles per wave, only for the
 // 256-feature q8_K epilogue)
 constexpr tile_cfg k_tiles[] = {{4, 2, 2, 2}, {2, 4, 3, 1}, {2, 4, 2, 1}, {4, 2, 1, 2}, {2, 4, 1, 1}, {4, 2, 1, 1}, {4, 2, 2, 1},
                                 {8, 1, 1, 2}, {4, 2, 3, 1}, {2, 2, 1, 1}};
+constexpr int FORCEABLE_TILES = 9;   // the hook's indices; the 64x64 tile runs by the rule alone
 // relative efficiency of one workgroup tile (larger tiles re-read less from L2 and LDS)
 constexpr double k_tile_eff[] = {1.0, 0.95, 0.85, 0.85, 0.65, 0.66, 0.8, 0.8, 0.9, 0.54};
 
@@ -1563,7 +1567,7 @@ int gemm_force_split(int split) {
 }
 
 int gemm_force_tile(int index) {
-    if (index >= (int) (sizeof(k_tiles) / sizeof(k_tiles[0]))) return -1;
+    if (index >= FORCEABLE_TILES) return -1;
     g_force_tile.store(index < 0 ? -1 : index);
     return 0;
 }

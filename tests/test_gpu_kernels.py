@@ -369,6 +369,30 @@ def test_matmul_f16_split_parts(jlib, oracle, shape):
     assert len(ran) >= 3
 
 
+# few rows, where the launcher takes the 64 x 64 tile (four waves): edges of its 64 tokens, one to 24 stages, a half stage
+@pytest.mark.parametrize("gtype", [gguf.GGML_Q8_0, gguf.GGML_Q4_0, gguf.GGML_Q4_K, gguf.GGML_F16])
+@pytest.mark.parametrize("M,N,K", [(2, 128, 256), (63, 128, 512), (65, 256, 768), (129, 384, 320), (197, 384, 1536), (576, 768, 3072)])
+def test_matmul_few_rows(jlib, oracle, gtype, M, N, K):
+    if gtype == gguf.GGML_Q4_K and K % 256:
+        K = 256
+    rng = np.random.default_rng(M + K + gtype)
+    w = (rng.standard_normal((N, K)) * 0.02).astype(np.float32)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    bias = (rng.standard_normal(N) * 0.02).astype(np.float32)
+    raw = w.astype(np.float16).view(np.uint8) if gtype == gguf.GGML_F16 else gguf.quantize(gtype, w)
+    want = _mul_mat_as_gpu(jlib, oracle, gtype, raw, N, K, x, bias)
+    dw, dx, db = dev(raw.reshape(-1)), dev(x), dev(bias)
+    y = torch.full((M, N), float("nan"), dtype=torch.float32, device="cuda")
+    torch.cuda.synchronize()
+    rc = jlib.lib().jepa_amd_matmul(0, gtype, dw.data_ptr(), N, K, db.data_ptr(), dx.data_ptr(), M, y.data_ptr(), 1, None)
+    assert rc == 0, jlib.error_text()
+    got = host(y)
+    if gtype != gguf.GGML_F16:
+        np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
+    else:   # another order of K f32 sums
+        assert np.abs(got - want).max() <= 2e-5 * np.abs(want).max()
+
+
 # workgroup tiles of the MFMA GEMM (weight rows x tokens), by index
 TILES = {0: (256, 128), 1: (192, 128), 2: (128, 128), 3: (128, 128), 4: (64, 128), 5: (128, 64), 6: (256, 64), 7: (256, 64),
          8: (384, 64)}
