@@ -7,7 +7,8 @@
 // the context; each slot has an event that says when its last copy is done. The device side of a copy is
 // a kernel that reads or writes the pinned memory: at this size hipMemcpyAsync costs more per piece
 // (1.77 MB up / down, CPU copies included: 64 / 64 us against 72 / 89; 4 MB 126 / 129 against 153 / 192;
-// pieces of 256 KB and 1 MB are slower for the kernel).
+// pieces of 256 KB and 1 MB are slower for the kernel). Where the system grants no pinned memory the copies go
+// through the runtime's staging buffer.
 #pragma once
 #include "common.h"
 
@@ -15,6 +16,7 @@
 
 #include <algorithm>
 #include <cstddef>
+#include <cstdlib>
 #include <cstring>
 
 // n bytes (a multiple of 4, both ends 4-byte aligned) between memory the device can address (misc.hip)
@@ -34,7 +36,7 @@ struct host_staging {
     // to p. The source is read before the call returns.
     template <class F>
     bool upload(void * dst, size_t bytes, hipStream_t s, F && fill) {
-        if (!ready()) return false;
+        if (!ready()) return upload_pageable(dst, bytes, s, fill);
         for (size_t at = 0; at < bytes; at += SLOT) {
             const size_t n = std::min(SLOT, bytes - at);
             const int k = next++ % N;
@@ -52,7 +54,8 @@ struct host_staging {
 
     // src[0, bytes) on the device to host memory, after the work enqueued on s; returns when dst is whole
     bool download(void * dst, const void * src, size_t bytes, hipStream_t s) {
-        if (!ready()) return false;
+        if (!ready())
+            return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s) == hipSuccess && hipStreamSynchronize(s) == hipSuccess;
         const size_t pieces = (bytes + SLOT - 1) / SLOT;
         const unsigned first = next;
         auto ask = [&](size_t i) {
@@ -79,18 +82,30 @@ private:
     bool busy[N] = {};
     unsigned next = 0;
 
+    // the slots are there (made on first use); if not, the next call asks again
     bool ready() {
         if (mem) return true;
         std::lock_guard<std::recursive_mutex> lk(jepa_hip_mutex());
+        bool ok = true;
         for (hipEvent_t & e : done)
-            if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) { e = nullptr; return false; }
+            if (ok && !e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) { e = nullptr; ok = false; }
         void * p = nullptr;
-        if (hipHostMalloc(&p, SLOT * N, hipHostMallocDefault) != hipSuccess) {
-            jepa_log("jepa: hipHostMalloc(%zu) failed\n", SLOT * N);
-            return false;
+        ok = ok && hipHostMalloc(&p, SLOT * N, hipHostMallocDefault) == hipSuccess;
+        if (ok) mem = (unsigned char *) p;
+        else (void) hipGetLastError();   // (the forward takes an error left on the thread for one of its launches)
+        return ok;
+    }
+    template <class F>
+    static bool upload_pageable(void * dst, size_t bytes, hipStream_t s, F && fill) {
+        unsigned char * p = (unsigned char *) malloc(std::min(SLOT, bytes));
+        bool ok = p != nullptr;
+        for (size_t at = 0; ok && at < bytes; at += SLOT) {
+            const size_t n = std::min(SLOT, bytes - at);
+            fill(p, at, n);
+            ok = hipMemcpyAsync((char *) dst + at, p, n, hipMemcpyHostToDevice, s) == hipSuccess && hipStreamSynchronize(s) == hipSuccess;
         }
-        mem = (unsigned char *) p;
-        return true;
+        free(p);
+        return ok;
     }
     bool settle(int k) {   // slot k is free again
         if (busy[k] && hipEventSynchronize(done[k]) != hipSuccess) return false;
