@@ -382,11 +382,15 @@ __global__ void k_copy_bytes(const uint32_t * __restrict__ src, uint32_t * __res
     for (int64_t i = 4 * n4 + i0; i < n; i += step) dst[i] = src[i];
 }
 
-void launch_copy_bytes(const void * src, void * dst, size_t n, hipStream_t s) {
-    const bool wide = (((uintptr_t) src | (uintptr_t) dst) & 15) == 0;
+// (the launch's own status: hipGetLastError would also report what an earlier call left on the thread)
+bool launch_copy_bytes(const void * src, void * dst, size_t n, hipStream_t s) {
+    bool wide = (((uintptr_t) src | (uintptr_t) dst) & 15) == 0;
     const size_t items = (n / 4 + 3) / 4;
-    if (n >= 4) k_copy_bytes<<<(unsigned) std::min<size_t>(512, (items + 255) / 256), 256, 0, s>>>((const uint32_t *) src, (uint32_t *) dst,
-                                                                                                 (int64_t) (n / 4), wide);
+    int64_t words = (int64_t) (n / 4);
+    if (words == 0) return true;
+    void * args[] = {&src, &dst, &words, &wide};
+    return hipLaunchKernel((const void *) k_copy_bytes, dim3((unsigned) std::min<size_t>(512, (items + 255) / 256)), dim3(256), args, 0, s) ==
+           hipSuccess;
 }
 
 // [n_rows][hd] RoPE tables (signed sine) of the tokens ids, from the rows of each axis (rope3d_axis_tables: the

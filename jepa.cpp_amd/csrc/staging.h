@@ -19,8 +19,9 @@
 #include <cstdlib>
 #include <cstring>
 
-// n bytes (a multiple of 4, both ends 4-byte aligned) between memory the device can address (misc.hip)
-void launch_copy_bytes(const void * src, void * dst, size_t n, hipStream_t s);
+// n bytes (a multiple of 4, both ends 4-byte aligned) between memory the device can address (misc.hip); false: not
+// launched
+bool launch_copy_bytes(const void * src, void * dst, size_t n, hipStream_t s);
 
 struct host_staging {
     static constexpr size_t SLOT = 512 * 1024;
@@ -43,8 +44,7 @@ struct host_staging {
             if (!settle(k)) return false;
             unsigned char * p = mem + (size_t) k * SLOT;
             fill(p, at, n);
-            launch_copy_bytes(p, (char *) dst + at, n, s);
-            if (!mark(k, s)) return false;
+            if (!launch_copy_bytes(p, (char *) dst + at, n, s) || !mark(k, s)) return false;
         }
         return true;
     }
@@ -61,8 +61,7 @@ struct host_staging {
         auto ask = [&](size_t i) {
             const int k = (int) ((first + i) % N);
             if (!settle(k)) return false;
-            launch_copy_bytes((const char *) src + i * SLOT, mem + (size_t) k * SLOT, std::min(SLOT, bytes - i * SLOT), s);
-            return mark(k, s);
+            return launch_copy_bytes((const char *) src + i * SLOT, mem + (size_t) k * SLOT, std::min(SLOT, bytes - i * SLOT), s) && mark(k, s);
         };
         for (size_t i = 0; i < std::min<size_t>(N, pieces); i++)
             if (!ask(i)) return false;
@@ -113,6 +112,8 @@ private:
         return true;
     }
     bool mark(int k, hipStream_t s) {   // slot k is in use until the work enqueued on s so far is done
-        return busy[k] = hipGetLastError() == hipSuccess && hipEventRecord(done[k], s) == hipSuccess;
+        busy[k] = hipEventRecord(done[k], s) == hipSuccess;
+        if (!busy[k]) (void) hipStreamSynchronize(s);
+        return busy[k];
     }
 };

@@ -14,7 +14,7 @@ namespace {
 std::vector<std::function<void()>> g_queue;       // the stream's work in order
 size_t g_done = 0;                                 // entries already run
 std::vector<size_t> g_events;                      // queue position each event stands for
-bool g_refuse_pinned = false;
+bool g_refuse_pinned = false, g_refuse_launch = false;
 hipError_t g_last = hipSuccess;
 int g_kernels = 0, g_memcpys = 0;
 
@@ -58,9 +58,11 @@ std::recursive_mutex & jepa_hip_mutex() {
     static std::recursive_mutex m;
     return m;
 }
-void launch_copy_bytes(const void * s, void * d, size_t n, hipStream_t) {
+bool launch_copy_bytes(const void * s, void * d, size_t n, hipStream_t) {
+    if (g_refuse_launch) return false;
     g_kernels++;
     g_queue.push_back([=] { memcpy(d, s, n); });
+    return true;
 }
 
 namespace {
@@ -101,6 +103,19 @@ int main(int argc, char ** argv) {
         CHECK(g_last == hipSuccess);      // nothing left behind for the forward's own check
         g_refuse_pinned = false;          // granted later: the slots are used
         CHECK(round_trips(true) == 0 && g_kernels > 0);
+        return 0;
+    }
+    if (c == "stale") {
+        CHECK(round_trips(true) == 0);
+        g_last = hipErrorInvalidDevice;   // left by some earlier call of the program
+        CHECK(round_trips(true) == 0);
+        g_last = hipErrorInvalidDevice;
+        CHECK(round_trips(false) == 0);
+        g_last = hipSuccess;              // a launch that fails is still reported
+        g_refuse_launch = true;
+        host_staging st;
+        unsigned char a[8] = {}, b[8];
+        CHECK(!st.upload(b, a, 8, nullptr) && !st.download(a, b, 8, nullptr));
         return 0;
     }
     fprintf(stderr, "no case %s\n", c.c_str());

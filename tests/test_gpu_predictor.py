@@ -117,3 +117,18 @@ def test_vitl16_predictor_q8_0(jlib, oracle, models_dir):
     print(f"vitl16 predictor 1024 + 1024 rows: {ctx.last_compute_ms:.3f} ms")
     want, want16 = _oracle_pair(oracle, path, enc, c, t, 1024)
     check(got, want, "vitl16 predictor", want16)
+
+
+def test_error_left_on_the_thread(jlib, models_dir):
+    """An error that an earlier HIP call left on the calling thread (here a device that is not there) belongs to
+    that call: the predictor's transfers are not refused for it."""
+    cfg = _tiny("vjepa2", "q8_0")
+    ctx = jlib.Context(jlib.Model(forge.cached_model(cfg, models_dir)))
+    enc = np.random.default_rng(3).standard_normal((32, cfg.embed_dim)).astype(np.float32)
+    want = ctx.predict(enc, np.arange(12), np.arange(12, 32))
+    assert jlib.lib().hipSetDevice(9999) != 0
+    try:
+        got = ctx.predict(enc, np.arange(12), np.arange(12, 32))
+    finally:
+        jlib.lib().hipGetLastError()
+    np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))

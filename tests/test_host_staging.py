@@ -19,6 +19,7 @@ def program(tmp_path_factory):
 @pytest.mark.parametrize("case", [
     "slots",       # transfers of one to many pieces: no slot is filled again or read before its copy is done
     "refused",     # no pinned memory: the same transfers through the runtime's copies, and no error left on the thread
+    "stale",       # an error that an earlier call left on the thread does not refuse a transfer; a failed launch does
 ])
 def test_staging(program, case):
     r = subprocess.run([program, case], capture_output=True, text=True, timeout=60)
