@@ -541,6 +541,7 @@ int64_t encode_host(jepa_context * ctx, const jepa_input * in, float * out_host,
             jepa_log("jepa: output download failed\n");
             r = -1;
         }
+        if (r <= 0) hipStreamSynchronize(ctx->stream);   // the caller's input may still be read
     } else {
         jepa_log("jepa: input upload failed\n");
     }

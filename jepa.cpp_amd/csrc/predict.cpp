@@ -115,8 +115,10 @@ bool upload_rope(jepa_context * ctx, const rope3d_params & rp, const int32_t * i
         w.rope_src_cap = cap;
     }
     char * dev = (char *) w.rope_src;
-    if (!ctx->staging->upload(dev, ids, nb, ctx->stream) || !ctx->staging->upload(dev + nb, c.data(), tb, ctx->stream) ||
-        !ctx->staging->upload(dev + nb + tb, sn.data(), tb, ctx->stream)) return false;
+    auto put = [&](void * dst, const void * src, size_t bytes) {   // (read before the call returns: the vectors end here)
+        return ctx->staging->upload(dst, bytes, ctx->stream, [&](void * p, size_t at, size_t n) { memcpy(p, (const char *) src + at, n); });
+    };
+    if (!put(dev, ids, nb) || !put(dev + nb, c.data(), tb) || !put(dev + nb + tb, sn.data(), tb)) return false;
     launch_rope_rows((const int32_t *) dev, (const float *) (dev + nb), (const float *) (dev + nb + tb), N, rp.head_dim,
                      rope3d_axis_dim(rp.head_dim), rp.grid_t, rp.grid_h, rp.grid_w, w.rope_c, w.rope_s, ctx->stream);
     return true;

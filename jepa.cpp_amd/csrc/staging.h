@@ -1,14 +1,22 @@
 // staging.h - host <-> device transfers of a context's host-buffer calls through its own pinned memory.
 //
-// A copy from or to pageable memory goes through the runtime's staging buffer, one piece after the
-// other, and the call waits for it: 4 MB took 137 us up and 255 us down where the same bytes take 86 us
-// between pinned memory and the device (measured, one MI355X box). Here the CPU copy of one piece
-// runs while the one before is on its way. Eight slots of 512 KB, made on first use and freed with
-// the context; each slot has an event that says when its last copy is done. The device side of a copy is
-// a kernel that reads or writes the pinned memory: at this size hipMemcpyAsync costs more per piece
-// (1.77 MB up / down, CPU copies included: 64 / 64 us against 72 / 89; 4 MB 126 / 129 against 153 / 192;
-// pieces of 256 KB and 1 MB are slower for the kernel). Where the system grants no pinned memory the copies go
-// through the runtime's staging buffer.
+// A copy to pageable memory goes through the runtime's staging buffer, one piece after the other, and the call
+// waits for it. Here the CPU copy of one piece runs while the one before is on its way: eight slots of 512 KB,
+// made on first use and freed with the context; each slot has an event that says when its last copy is done. The
+// device side of a copy is a kernel that reads or writes the pinned memory: hipMemcpyAsync costs more per piece.
+// Where the system grants no pinned memory the copies go through the runtime.
+//
+// us of one transfer, hipMemcpyAsync / slots, waited for (hot: the same host buffer each time; cold: more buffers
+// than the CPU's cache holds):
+//   down, cold     64 KB 36 / 14, 512 KB 31 / 34, 2 MB 122 / 117, 4 MB 243 / 222, 16 MB 979 / 867; hot 4 MB 237 / 134
+//   up, hot        16 KB 18 / 13, 64 KB 33 / 14, 256 KB 15 / 20 (one box 109 / 20), 600 KB 27 / 37, 2 MB 80 / 89,
+//                  4 MB 133 / 157, 16 MB 460 / 570
+//   up, cold       600 KB 32 / 42, 2 MB 102 / 93, 4 MB 179 / 164, 16 MB 608 / 576
+//   up, registered 600 KB 20 / 36, 4 MB 83 / 157, 16 MB 301 / 564
+// So every download takes the slots, and so do uploads of at most one slot and uploads that gather their source.
+// Above one slot the runtime pins the source's pages and copies from there: no CPU copy, which is what bounds the
+// slots (~30 GB/s). Memory that the runtime already knows (pinned, registered, managed, device) is copied from
+// where it is at any size.
 #pragma once
 #include "common.h"
 
@@ -34,7 +42,7 @@ struct host_staging {
     }
 
     // dst[0, bytes) on the device, enqueued on s; fill(p, at, n) writes bytes [at, at + n) of the source
-    // to p. The source is read before the call returns.
+    // to p, before the call returns
     template <class F>
     bool upload(void * dst, size_t bytes, hipStream_t s, F && fill) {
         if (!ready()) return upload_pageable(dst, bytes, s, fill);
@@ -48,7 +56,9 @@ struct host_staging {
         }
         return true;
     }
+    // the source may be read until the work enqueued on s is done
     bool upload(void * dst, const void * src, size_t bytes, hipStream_t s) {
+        if (bytes > SLOT || known(src)) return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s) == hipSuccess;
         return upload(dst, bytes, s, [&](void * p, size_t at, size_t n) { memcpy(p, (const char *) src + at, n); });
     }
 
@@ -93,6 +103,13 @@ private:
         if (ok) mem = (unsigned char *) p;
         else (void) hipGetLastError();   // (the forward takes an error left on the thread for one of its launches)
         return ok;
+    }
+    // memory of the HIP runtime's own: pinned or registered host memory, managed or device memory
+    static bool known(const void * p) {
+        hipPointerAttribute_t a{};
+        if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type != hipMemoryTypeUnregistered;
+        (void) hipGetLastError();
+        return false;
     }
     template <class F>
     static bool upload_pageable(void * dst, size_t bytes, hipStream_t s, F && fill) {

@@ -17,6 +17,7 @@ std::vector<size_t> g_events;                      // queue position each event 
 bool g_refuse_pinned = false, g_refuse_launch = false;
 hipError_t g_last = hipSuccess;
 int g_kernels = 0, g_memcpys = 0;
+std::vector<std::pair<const unsigned char *, size_t>> g_known;   // memory the runtime knows
 
 void run_to(size_t n) {
     for (; g_done < n; g_done++) g_queue[g_done]();
@@ -44,6 +45,13 @@ hipError_t hipGetLastError() { const hipError_t e = g_last; g_last = hipSuccess;
 hipError_t hipMemcpyAsync(void * d, const void * s, size_t n, hipMemcpyKind, hipStream_t) {
     g_memcpys++;
     g_queue.push_back([=] { memcpy(d, s, n); });
+    return hipSuccess;
+}
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t * a, const void * p) {
+    *a = {};
+    a->type = hipMemoryTypeUnregistered;
+    for (const auto & k : g_known)
+        if (p >= k.first && p < k.first + k.second) a->type = hipMemoryTypeHost;
     return hipSuccess;
 }
 }
@@ -74,8 +82,8 @@ std::vector<unsigned char> bytes_of(size_t n, unsigned seed) {
     return v;
 }
 
-// several transfers each way through one object, with pieces before and past the eight slots; the source of an
-// upload is overwritten as soon as the call returns
+// several transfers each way through one object, with pieces before and past the eight slots; the source of a
+// gathering upload, and of one that takes the slots, is overwritten as soon as the call returns
 int round_trips(bool plain) {
     host_staging st;
     const size_t slot = host_staging::SLOT;
@@ -85,6 +93,7 @@ int round_trips(bool plain) {
         std::vector<unsigned char> src = a, dev(n, 0), back(n, 0);
         if (plain) CHECK(st.upload(dev.data(), src.data(), n, nullptr));
         else CHECK(st.upload(dev.data(), n, nullptr, [&](void * p, size_t at, size_t k) { memcpy(p, src.data() + at, k); }));
+        if (plain) run_to(g_queue.size());
         std::fill(src.begin(), src.end(), 0xee);
         CHECK(st.download(back.data(), dev.data(), n, nullptr));
         CHECK(back == a);
@@ -102,7 +111,27 @@ int main(int argc, char ** argv) {
         CHECK(g_kernels == 0 && g_memcpys > 0);
         CHECK(g_last == hipSuccess);      // nothing left behind for the forward's own check
         g_refuse_pinned = false;          // granted later: the slots are used
+        g_kernels = 0;
         CHECK(round_trips(true) == 0 && g_kernels > 0);
+        return 0;
+    }
+    if (c == "direct") {
+        // one copy from where the source is: more than a slot, or memory the runtime knows, of any size
+        host_staging st;
+        const size_t slot = host_staging::SLOT;
+        std::vector<unsigned char> src = bytes_of(2 * slot, 5), dev(2 * slot, 0);
+        auto takes = [&](const unsigned char * p, size_t n, int kernels, int memcpys) {
+            g_kernels = g_memcpys = 0;
+            std::fill(dev.begin(), dev.end(), 0);
+            if (!st.upload(dev.data(), p, n, nullptr)) return false;
+            run_to(g_queue.size());
+            return g_kernels == kernels && g_memcpys == memcpys && memcmp(dev.data(), p, n) == 0;
+        };
+        CHECK(takes(src.data(), 4, 1, 0) && takes(src.data(), slot, 1, 0));
+        CHECK(takes(src.data(), slot + 4, 0, 1) && takes(src.data(), 2 * slot, 0, 1));
+        g_known.push_back({src.data() + slot, slot});
+        CHECK(takes(src.data() + slot, 4, 0, 1) && takes(src.data() + slot + 400, slot - 400, 0, 1));
+        CHECK(takes(src.data(), slot, 1, 0));
         return 0;
     }
     if (c == "stale") {

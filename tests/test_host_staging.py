@@ -19,6 +19,7 @@ def program(tmp_path_factory):
 @pytest.mark.parametrize("case", [
     "slots",       # transfers of one to many pieces: no slot is filled again or read before its copy is done
     "refused",     # no pinned memory: the same transfers through the runtime's copies, and no error left on the thread
+    "direct",      # uploads of more than one slot, and from memory the runtime knows, are one copy from where it is
     "stale",       # an error that an earlier call left on the thread does not refuse a transfer; a failed launch does
 ])
 def test_staging(program, case):
