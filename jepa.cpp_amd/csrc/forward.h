@@ -31,7 +31,6 @@ struct fwd_workspace {
     int n_ctx = 0, n_tgt = 0;
     float * pin = nullptr, * pout = nullptr;
     void * rope_src = nullptr;   // token ids, then the RoPE rows of each axis
-    size_t rope_src_cap = 0;
     act_view actC;
     // graph
     hipGraphExec_t exec = nullptr;

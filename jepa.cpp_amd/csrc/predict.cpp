@@ -77,6 +77,9 @@ rope3d_params pred_rope(const jepa_model * m, int64_t max_id) {
     return rp;
 }
 
+// rows of all axis tables for N tokens: each has a temporal position of its own at most
+size_t rope_axis_rows(const rope3d_params & rp, int64_t N) { return (size_t) N + rp.grid_h + rp.grid_w; }
+
 bool ensure_pred_workspace(jepa_context * ctx, int n_ctx, int n_tgt) {
     const jepa_model * m = ctx->model;
     const pred_hparams & p = m->hp.pred;
@@ -97,7 +100,8 @@ bool ensure_pred_workspace(jepa_context * ctx, int n_ctx, int n_tgt) {
                     ws_alloc(*w, (void **) &w->pin, (size_t) std::max(n_ctx, 1) * De * 4) &&
                     ws_alloc_act(*w, w->actC, std::max(n_ctx, 1), De) &&
                     ws_alloc(*w, (void **) &w->pout, (size_t) n_tgt * pr.proj.n_out * 4) &&
-                    ws_alloc(*w, (void **) &w->rope_c, (size_t) N * b.hd * 4) && ws_alloc(*w, (void **) &w->rope_s, (size_t) N * b.hd * 4);
+                    ws_alloc(*w, (void **) &w->rope_c, (size_t) N * b.hd * 4) && ws_alloc(*w, (void **) &w->rope_s, (size_t) N * b.hd * 4) &&
+                    ws_alloc(*w, &w->rope_src, (size_t) N * 4 + 2 * rope_axis_rows(pred_rope(m, 0), N) * rope3d_axis_dim(b.hd) * 4);
     if (!ok || hipStreamSynchronize(ctx->stream) != hipSuccess) { ctx->pws.reset(); return false; }
     return true;
 }
@@ -105,22 +109,18 @@ bool ensure_pred_workspace(jepa_context * ctx, int n_ctx, int n_tgt) {
 // the RoPE tables of the tokens ids into w.rope_c / w.rope_s
 bool upload_rope(jepa_context * ctx, const rope3d_params & rp, const int32_t * ids, int64_t N) {
     fwd_workspace & w = *ctx->pws;
+    std::vector<int32_t> times, place;
     std::vector<float> c, sn;
-    rope3d_axis_tables(rp, c, sn);
+    rope3d_compact(rp, ids, N, times, place);
+    rope3d_axis_tables(rp, times, c, sn);
     const size_t nb = (size_t) N * 4, tb = c.size() * 4;
-    if (w.rope_src_cap < nb + 2 * tb) {   // (the temporal rows grow with the largest id)
-        std::lock_guard<std::recursive_mutex> lk(jepa_hip_mutex());
-        const size_t cap = 2 * (nb + 2 * tb);
-        if (!ws_alloc(w, &w.rope_src, cap)) { w.rope_src_cap = 0; return false; }
-        w.rope_src_cap = cap;
-    }
     char * dev = (char *) w.rope_src;
     auto put = [&](void * dst, const void * src, size_t bytes) {   // (read before the call returns: the vectors end here)
         return ctx->staging->upload(dst, bytes, ctx->stream, [&](void * p, size_t at, size_t n) { memcpy(p, (const char *) src + at, n); });
     };
-    if (!put(dev, ids, nb) || !put(dev + nb, c.data(), tb) || !put(dev + nb + tb, sn.data(), tb)) return false;
+    if (!put(dev, place.data(), nb) || !put(dev + nb, c.data(), tb) || !put(dev + nb + tb, sn.data(), tb)) return false;
     launch_rope_rows((const int32_t *) dev, (const float *) (dev + nb), (const float *) (dev + nb + tb), N, rp.head_dim,
-                     rope3d_axis_dim(rp.head_dim), rp.grid_t, rp.grid_h, rp.grid_w, w.rope_c, w.rope_s, ctx->stream);
+                     rope3d_axis_dim(rp.head_dim), (int) times.size(), rp.grid_h, rp.grid_w, w.rope_c, w.rope_s, ctx->stream);
     return true;
 }
 

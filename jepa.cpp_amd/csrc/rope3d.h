@@ -20,8 +20,11 @@ struct rope3d_params {
 };
 
 int rope3d_axis_dim(int head_dim);
-// the rows of each axis, [dims[axis]][axis_dim] cosines and (unsigned) sines, t then h then w
-void rope3d_axis_tables(const rope3d_params & p, std::vector<float> & cos_out, std::vector<float> & sin_out);
+// the rows of each axis, [axis_dim] cosines and (unsigned) sines each: one per temporal position of `times`, then h,
+// then w
+void rope3d_axis_tables(const rope3d_params & p, const std::vector<int32_t> & times, std::vector<float> & cos_out, std::vector<float> & sin_out);
+// the temporal positions that occur among ids (tokens of the grid), and the ids on a grid of those positions alone
+void rope3d_compact(const rope3d_params & p, const int32_t * ids, int64_t n, std::vector<int32_t> & times, std::vector<int32_t> & compact_ids);
 // [n_rows, head_dim] tables; ids == nullptr means every token of the grid in T-major order
 void rope3d_tables(const rope3d_params & p, const int32_t * ids, int64_t n_rows, std::vector<float> & cos_out,
                    std::vector<float> & sin_out, bool signed_sin = true);

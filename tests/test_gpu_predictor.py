@@ -119,6 +119,27 @@ def test_vitl16_predictor_q8_0(jlib, oracle, models_dir):
     check(got, want, "vitl16 predictor", want16)
 
 
+def test_far_target_ids(jlib, oracle, models_dir):
+    """Target ids at the last temporal slices the predictor accepts, and slices out of order: the call needs the
+    RoPE rows of the slices that occur and takes no device memory for those between."""
+    import torch
+    cfg = _tiny("vjepa2", "q8_0")
+    path = forge.cached_model(cfg, models_dir)
+    ctx = jlib.Context(jlib.Model(path))
+    enc = np.random.default_rng(5).standard_normal((32, cfg.embed_dim)).astype(np.float32)
+    per = (cfg.img_size // cfg.patch) ** 2
+    c, near = np.arange(12), np.arange(12, 32)
+    first = ctx.predict(enc, c, near)
+    free = torch.cuda.mem_get_info()[0]
+    for slices in ([65535] * 20, list(range(40000, 40020)), [9000, 3, 1, 9000, 20000] * 4):
+        far = near % per + np.array(slices) * per
+        got = ctx.predict(enc, c, far)
+        want, want16 = _oracle_pair(oracle, path, enc, c, far, cfg.embed_dim)
+        check(got, want, f"slices {slices[:3]}", want16)
+        assert torch.cuda.mem_get_info()[0] == free
+    np.testing.assert_array_equal(ctx.predict(enc, c, near).view(np.uint32), first.view(np.uint32))
+
+
 def test_error_left_on_the_thread(jlib, models_dir):
     """An error that an earlier HIP call left on the calling thread (here a device that is not there) belongs to
     that call: the predictor's transfers are not refused for it."""
