@@ -166,11 +166,16 @@ int jepa_amd_copy(int device, const float * src_dev, float * dst_dev, int64_t n,
 /* Force the MFMA GEMM onto workgroup tile `index` for later launches whose n_out it divides; -1
  * restores the automatic choice. Process-wide (tests and tuning). Tiles (weight rows x tokens):
  * 0: 256x128, 1: 192x128, 2: 128x128, 3: 128x128 (other wave shape), 4: 64x128, 5: 128x64, 6: 256x64,
- * 7: 256x64 (other wave shape; only for the q8_K GELU epilogue), 8: 384x64 (4-bit q4_0 only). q4_K
+ * 7: 256x64 (other wave shape; only for the q8_K GELU epilogue), 8: 384x64 (4-bit q4_0 only); 9, 64x64 of
+ * four waves, runs by the automatic choice alone and is refused here. q4_K
  * weights run tiles 2, 3, 5, 6 and 7, 4-bit q4_0 (rows a multiple of 128) tiles 0, 2, 3, 5, 6, 7 and 8;
  * a tile a launch cannot take leaves that launch on the automatic choice.
  * Returns 0, or -1 for an index past the table. */
 int jepa_amd_gemm_tile(int index);
+/* The tile (0 to 9 above) a GEMM of this shape takes with the plain f32 epilogue, the residual one or any that
+ * does not need 256 features; -1 for f32 weights and types without a GEMM. One row of q8_0 codes has a
+ * kernel of its own where no tile or split is forced. No device work. */
+int jepa_amd_gemm_tile_of(int wtype, int64_t n_out, int64_t n_in, int64_t n_rows);
 
 #ifdef __cplusplus
 }

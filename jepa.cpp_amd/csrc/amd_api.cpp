@@ -284,6 +284,11 @@ extern "C" int jepa_amd_gemm_tile(int index) {
     return 0;
 }
 
+extern "C" int jepa_amd_gemm_tile_of(int wtype, int64_t n_out, int64_t n_in, int64_t n_rows) {
+    const int wf = weight_format(wtype, n_in);
+    return wf < 0 || wf == W_F32 || n_out <= 0 || n_in <= 0 || n_rows <= 0 ? -1 : gemm_tile_for(wf, n_out, n_in, n_rows);
+}
+
 extern "C" int jepa_amd_attention(int device, const float * qkv, int64_t n_items, int64_t n_tok, int n_head, int hd,
                                   const float * rope_c, const float * rope_s, int n_prefix, int64_t tokens_per_slot, int out_type,
                                   void * out) {

@@ -1349,9 +1349,16 @@ bool tile_ok(int wf, int c) {
     return c != 8;
 }
 
+// The 64x64 tile saves time per launch (fewer rows to copy before the first step and to store after the last)
+// and loses some per K stage, with 4-bit q4_0 codes, whose unpacking four waves share: from about 12 stages
+// of 128 columns on the 128x64 tile is as fast or faster. us for 128x64 / 64x64, q4_0 64 rows: 1024 x 1024
+// 9.4 / 8.9, 384 x 1536 11.6 / 11.3, 768 x 3072 18.9 / 18.8 (2 rows 18.4 / 19.1), 1024 x 4096 23.9 / 24.4, 1408 x 6144
+// 33.5 / 34.4; one shape of the longer ones gains, 400 rows of 1408 x 6144 39.4 / 36.2.
+constexpr int64_t Q40_SMALL_TILE_MAX_K = 2048;
+
 // The tile with the least estimated time: whole waves of workgroups over the CUs (one workgroup per
 // CU) times the work of one tile, discounted by the tile's efficiency. Only tiles dividing N.
-int pick_tile(int wf, int64_t N, int64_t M, int need_bn = 0, int split = 1) {
+int pick_tile(int wf, int64_t N, int64_t K, int64_t M, int need_bn = 0, int split = 1) {
     const int f = g_force_tile.load();
     const int nt = (int) (sizeof(k_tiles) / sizeof(k_tiles[0]));
     const auto bn_of = [](int c) { return 32 * k_tiles[c].wn * k_tiles[c].ti; };
@@ -1363,7 +1370,7 @@ int pick_tile(int wf, int64_t N, int64_t M, int need_bn = 0, int split = 1) {
     for (int c = 0; c < nt; c++) {
         const int64_t bn = 32 * k_tiles[c].wn * k_tiles[c].ti, bm = 32 * k_tiles[c].wm * k_tiles[c].tj;
         if (N % bn || (need_bn && bn != need_bn) || (c == 7 && need_bn != 256)) continue;
-        if (!tile_ok(wf, c)) continue;
+        if (!tile_ok(wf, c) || (c == 9 && wf == W_Q40 && K > Q40_SMALL_TILE_MAX_K)) continue;
         const int64_t t = (N / bn) * ((M + bm - 1) / bm) * split;
         const double waves = (double) ((t + cus - 1) / cus);
         // q4_K unpacks a wave's weight operand once for its TJ token tiles: tiles with two token tiles
@@ -1463,7 +1470,7 @@ void dispatch_mfma(kargs a, hipStream_t s, const gemm_split_ws * sw) {
     const bool can_split = sw && sw->part && sw->cnt && (a.ep.kind == EPI_RESID || a.ep.kind == EPI_F32);
     a.split = can_split && WF != W_F16 ? gemm_split_for(WF, a.N, a.K) : 1;
     a.part = nullptr; a.cnt = nullptr;
-    const int c = pick_tile(WF, a.N, a.M, a.ep.kind == EPI_GELU_Q8_K ? 256 : 0, a.split);
+    const int c = pick_tile(WF, a.N, a.K, a.M, a.ep.kind == EPI_GELU_Q8_K ? 256 : 0, a.split);
     if (c < 0) {
         jepa_log("jepa: internal error: no 256-wide GEMM tile for the q8_K epilogue (N = %lld)\n", (long long) a.N);
         return;
@@ -1559,6 +1566,8 @@ void launch_gemm(const dev_linear & W, const act_view & X, int64_t M, const gemm
         case W_Q4K: dispatch_mfma<W_Q4K>(a, s, sw); break;
     }
 }
+
+int gemm_tile_for(int wf, int64_t N, int64_t K, int64_t M) { return pick_tile(wf, N, K, M, 0, wf == W_F16 ? 1 : gemm_split_for(wf, N, K)); }
 
 int gemm_force_split(int split) {
     // int8 / 4-bit weights: 1 or 2 halves; f16 weights: 1 to 4 parts (f16_split)

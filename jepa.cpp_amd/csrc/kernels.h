@@ -76,6 +76,8 @@ bool launch_gemv_q8(const dev_linear & W, const act_view & X, const gemm_epi & e
 // only, so that the summation order of an output never depends on the number of rows (f16 weights:
 // chosen per launch from the tile count, 1 here)
 int gemm_split_for(int wf, int64_t N, int64_t K);
+// workgroup tile (index of gemm.hip's table) a GEMM with the plain f32 epilogue runs; host only
+int gemm_tile_for(int wf, int64_t N, int64_t K, int64_t M);
 
 // LayerNorm (ggml_norm + affine) of x [M][D] written in `out` format; w/b may be null (no affine).
 // out.fmt A_F32 writes f32 rows into out.q. When normalize == false the rows are only quantized.

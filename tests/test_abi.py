@@ -102,3 +102,17 @@ def test_versions_and_defaults(L):
 def test_gemm_tile_hook_is_host_only(L):
     assert L.jepa_amd_gemm_tile(99) == -1
     assert L.jepa_amd_gemm_tile(-1) == 0
+
+
+# the 64 x 64 tile (9) of few rows: 4-bit q4_0 codes take it up to 16 stages of 128 columns, where it was measured
+# faster; the other formats at any K; and never where the launch has more tiles than there are CUs to take them
+@pytest.mark.parametrize("rows,n_out,n_in,q40,others", [
+    (2, 768, 768, 9, 9), (197, 384, 1536, 9, 9), (256, 1024, 1024, 9, 9), (64, 1024, 2048, 9, 9), (2, 768, 3072, 5, 9), (33, 1024, 4096, 5, 9),
+    (256, 1408, 6144, 5, 9), (1024, 1024, 4096, 5, 9),
+])
+def test_small_gemm_tile_rule(L, rows, n_out, n_in, q40, others):
+    assert L.jepa_amd_gemm_tile_of(2, n_out, n_in, rows) == q40
+    assert L.jepa_amd_gemm_tile_of(8, n_out, n_in, rows) == others
+    assert L.jepa_amd_gemm_tile_of(1, n_out, n_in, rows) == others
+    assert L.jepa_amd_gemm_tile_of(8, 4096, 1024, 2048) != 9
+    assert L.jepa_amd_gemm_tile_of(0, n_out, n_in, rows) == -1
