@@ -171,6 +171,28 @@ def test_qkv_rope_rows_on_every_tile(jlib, oracle, models_dir, ftype, tiles, n_r
         assert d.size == 0, (t, len(d), d[:4].tolist(), float(np.abs(y - got).max()))
 
 
+@pytest.mark.parametrize("ftype,ffn", [("q8_0", 1024), ("q4_0", 1024), ("q4_k", 2048), ("f16", 1024)])
+def test_small_tile_in_a_block(jlib, models_dir, ftype, ffn):
+    """Blocks whose four GEMMs take the 64 x 64 tile by the automatic choice (216 rows; QKV with RoPE, its rows copied
+    early for q8_0 and q4_0, residuals with layer scale, fc2 of q4_K in two K halves) give the bits of the same
+    blocks on the 128 x 64 tile."""
+    cfg = forge.tiny("vjepa2", ftype, embed_dim=512, n_head=8, ffn_dim=ffn, ln_random=True, layer_scale=True)
+    L = jlib.lib()
+    gt = {"q8_0": 8, "q4_0": 2, "q4_k": 12, "f16": 1}[ftype]
+    for n_out, n_in in ((1536, 512), (512, 512), (ffn, 512), (512, ffn)):
+        assert L.jepa_amd_gemm_tile_of(gt, n_out, n_in, 216) == 9
+    m = jlib.Model(forge.cached_model(cfg, models_dir))
+    x = inputs.make_input(3, 4, 96, 96, seed=3)
+    got = jlib.Context(m).encode(x)
+    assert L.jepa_amd_gemm_tile(5) == 0
+    try:
+        want = jlib.Context(m).encode(x)
+    finally:
+        L.jepa_amd_gemm_tile(-1)
+    assert got.shape == (216, 512) and np.isfinite(got).all()
+    np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
 @pytest.mark.parametrize("parts", ["q8_0+b,f16+b,q8_0+b", "q4_0+b,q8_0,q8_0+b"])
 def test_qkv_rope_rows_separate_parts(jlib, oracle, models_dir, parts):
     """Separate q / k / v linears of width 512 (K = 512: four stages) whose types differ, so each runs as
@@ -240,6 +262,35 @@ def test_graph_replay_equals_direct(jlib, models_dir):
     direct = ctx.encode(x)
     for a in again + [direct]:
         np.testing.assert_array_equal(a.view(np.uint32), first.view(np.uint32))
+
+
+@pytest.mark.parametrize("family,shape,cap", [("vjepa2", (2, 3, 4, 64, 64), 0), ("hfvit", (5, 3, 1, 64, 64), 2), ("ijepa", (1, 3, 1, 112, 112), 0)])
+def test_encode_device_with_new_buffers(jlib, models_dir, family, shape, cap):
+    """One context, one captured graph, several inputs and outputs each in a buffer of its own, in turn (5 images of a
+    context that takes 2 at a time among them): every call equals the same input without the graph, and no call
+    writes an output of another."""
+    import torch
+    m = jlib.Model(forge.cached_model(forge.tiny(family, "q8_0"), models_dir))
+    ctx, plain = jlib.Context(m), jlib.Context(m)
+    plain.set_graph(False)
+    for c in (ctx, plain):
+        jlib.lib().jepa_context_set_max_batch(c.ptr, cap)
+    rows = shape[0] * m.token_grid(*shape[2:])
+    want = [plain.encode(inputs.make_input(shape[0], *shape[2:], seed=i)) for i in range(3)]
+    ins = [torch.from_numpy(inputs.make_input(shape[0], *shape[2:], seed=i)).cuda() for i in range(3)]
+    outs = [torch.full((rows, m.dim), float("nan"), device="cuda") for _ in range(3)]
+    torch.cuda.synchronize()
+    for k, i in enumerate((0, 1, 2, 1, 0, 2)):
+        if k >= 3:
+            outs[i].fill_(float("nan"))
+            torch.cuda.synchronize()
+        ctx.encode_device(ins[i].data_ptr(), shape, outs[i].data_ptr(), outs[i].numel())
+        for j in range(3):
+            got = outs[j].cpu().numpy()
+            if k < 3 and j > i:
+                assert np.isnan(got).all()
+            else:
+                np.testing.assert_array_equal(got.view(np.uint32), want[j].view(np.uint32), err_msg=f"call {k}, output {j}")
 
 
 def test_vits16_f16_full(jlib, oracle, models_dir):

@@ -375,6 +375,7 @@ def test_matmul_f16_split_parts(jlib, oracle, shape):
 def test_matmul_few_rows(jlib, oracle, gtype, M, N, K):
     if gtype == gguf.GGML_Q4_K and K % 256:
         K = 256
+    assert jlib.lib().jepa_amd_gemm_tile_of(gtype, N, K, M) == (5 if gtype == gguf.GGML_Q4_0 and K > 2048 else 9)
     rng = np.random.default_rng(M + K + gtype)
     w = (rng.standard_normal((N, K)) * 0.02).astype(np.float32)
     x = rng.standard_normal((M, K)).astype(np.float32)
@@ -391,6 +392,33 @@ def test_matmul_few_rows(jlib, oracle, gtype, M, N, K):
         np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
     else:   # another order of K f32 sums
         assert np.abs(got - want).max() <= 2e-5 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("gtype,out_types", [(gguf.GGML_Q8_0, (0, 1, 8)), (gguf.GGML_Q4_0, (0, 8)), (gguf.GGML_Q4_K, (0, 8)), (gguf.GGML_F16, (0, 1, 8))])
+@pytest.mark.parametrize("M,N,K", [(2, 128, 256), (65, 384, 768), (389, 768, 1536)])
+def test_small_tile_gelu_equals_large_tile(jlib, gtype, out_types, M, N, K):
+    """The automatic choice for few rows, the 64 x 64 tile of four waves, writes the bytes of the 128 x 64 tile of
+    eight through each GELU epilogue (both sum an output's K steps in one order)."""
+    L = jlib.lib()
+    assert L.jepa_amd_gemm_tile_of(gtype, N, K, M) == 9
+    rng = np.random.default_rng(M + gtype)
+    w = (rng.standard_normal((N, K)) * 0.05).astype(np.float32)
+    w[32:64] = 0.0
+    raw = w.astype(np.float16).view(np.uint8) if gtype == gguf.GGML_F16 else gguf.quantize(gtype, w)
+    dw, dx, db = dev(raw.reshape(-1)), dev(rng.standard_normal((M, K)).astype(np.float32)), dev(rng.standard_normal(N).astype(np.float32))
+    for out_type in out_types:
+        got = []
+        for tile in (-1, 5):
+            out = torch.full((M * N * {0: 4, 1: 2}[out_type] if out_type < 8 else M * N // 32 * 34,), 77, dtype=torch.uint8, device="cuda")
+            torch.cuda.synchronize()
+            assert L.jepa_amd_gemm_tile(tile) == 0
+            try:
+                rc = L.jepa_amd_matmul_gelu(0, gtype, dw.data_ptr(), N, K, db.data_ptr(), dx.data_ptr(), M, out_type, out.data_ptr(), 1, None)
+            finally:
+                L.jepa_amd_gemm_tile(-1)
+            assert rc == 0, jlib.error_text()
+            got.append(host(out))
+        np.testing.assert_array_equal(got[0], got[1], err_msg=f"output type {out_type}")
 
 
 # workgroup tiles of the MFMA GEMM (weight rows x tokens), by index
