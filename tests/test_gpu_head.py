@@ -115,3 +115,36 @@ def test_vitl16_ssv2_head_q8_0(jlib, oracle, models_dir):
     print(f"vitl16 ssv2 head: {ctx.last_compute_ms:.3f} ms")
     want_p, want_l = oracle.head(path, rows, cfg.n_classes)
     check(got_p, got_l, want_p, want_l, "vitl16 ssv2 head")
+
+
+def test_one_row_linears_equal_the_tile_kernel(jlib, models_dir):
+    """One row of q8_0 codes through its own kernel inside whole calls, against the tile kernel (which a forced K split
+    of 1, otherwise without effect here, selects), bit for bit: the head's projections and MLP; a predictor of one
+    context and one target row, with the modality vector; one of a single row; blocks of a one-token image with
+    layer scale."""
+    L = jlib.lib()
+
+    def both(run):
+        got = run()
+        assert L.jepa_amd_gemm_split(1) == 0
+        try:
+            want = run()
+        finally:
+            L.jepa_amd_gemm_split(-1)
+        assert np.isfinite(got).all()
+        np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
+
+    rng = np.random.default_rng(23)
+    cfg = _tiny("q8_0")
+    ctx = jlib.Context(jlib.Model(forge.cached_model(cfg, models_dir)))
+    rows = rng.standard_normal((70, cfg.embed_dim)).astype(np.float32)
+    both(lambda: np.concatenate(ctx.head(rows)))
+    cfg = forge.tiny("vjepa2_1", "q8_0", ln_random=True, pred_dim=128, pred_layers=2, pred_ffn=512, w_std=0.08)
+    pred = jlib.Context(jlib.Model(forge.cached_model(cfg, models_dir)))
+    enc = rng.standard_normal((32, cfg.embed_dim)).astype(np.float32)
+    both(lambda: pred.predict(enc, [3], [7]))
+    both(lambda: pred.predict(enc, [], [7]))
+    one = jlib.Context(jlib.Model(forge.cached_model(forge.tiny("ijepa", "q8_0", img_size=14, layer_scale=True, ln_random=True), models_dir)))
+    x = inputs.make_input(1, 1, 14, 14, seed=2)
+    assert one.encode(x).shape[0] == 1
+    both(lambda: one.encode(x))

@@ -736,6 +736,12 @@ def test_attention_other_widths_stages(jlib, oracle, n_items, n_tok, n_prefix, s
     # f16 keys, values and weights: 2^-11 each (the bars of the other attention tests)
     assert np.abs(got - ref).max() / np.abs(ref).max() <= 1e-2
     assert ((got * ref).sum(1) / (np.linalg.norm(got, axis=1) * np.linalg.norm(ref, axis=1))).min() >= 0.9999
+    # the f16 output is the f32 output rounded
+    half = torch.full((n_items * n_tok, D), float("nan"), dtype=torch.float16, device="cuda")
+    torch.cuda.synchronize()
+    r = jlib.lib().jepa_amd_attention(0, dq.data_ptr(), n_items, n_tok, H, hd, None, None, n_prefix, slot, gguf.GGML_F16, half.data_ptr())
+    assert r == 0, jlib.error_text()
+    np.testing.assert_array_equal(host(half), host(out).astype(np.float16))
 
 
 @pytest.mark.parametrize("n_items,n_tok,H", [(1, 2048, 4), (2, 197, 6), (1, 65, 2)])
