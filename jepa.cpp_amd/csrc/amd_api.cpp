@@ -192,6 +192,14 @@ bool make_linear(dev_scope & d, const char * who, int wtype, const void * w, int
     return true;
 }
 
+// the input rows of a linear: f32 rows as they are, else converted
+bool make_act(dev_scope & d, act_view & a, const dev_linear & L, const float * x, int64_t n_rows) {
+    if (L.act() == A_F32) { a.fmt = A_F32; a.ld = L.n_in; a.q = (void *) x; return true; }
+    if (!alloc_act(d, a, L.act(), n_rows, L.n_in)) return false;
+    launch_rownorm_quant(x, n_rows, L.n_in, nullptr, nullptr, 0.0f, false, a, d.s);
+    return true;
+}
+
 }  // namespace
 
 extern "C" int jepa_amd_matmul(int device, int wtype, const void * w, int64_t n_out, int64_t n_in, const float * bias, const float * x,
@@ -202,8 +210,7 @@ extern "C" int jepa_amd_matmul(int device, int wtype, const void * w, int64_t n_
     dev_linear L;
     if (!make_linear(d, "jepa_amd_matmul", wtype, w, n_out, n_in, bias, L)) return -1;
     act_view a;
-    if (!alloc_act(d, a, L.act(), n_rows, n_in)) return -1;
-    launch_rownorm_quant(x, n_rows, n_in, nullptr, nullptr, 0.0f, false, a, d.s);
+    if (!make_act(d, a, L, x, n_rows)) return -1;
     gemm_split_ws sw;
     if (!alloc_split(d, sw, n_rows)) return -1;
     gemm_epi ep;
@@ -242,8 +249,7 @@ extern "C" int jepa_amd_matmul_gelu(int device, int wtype, const void * w, int64
         return -1;
     }
     act_view a;
-    if (!alloc_act(d, a, L.act(), n_rows, n_in)) return -1;
-    launch_rownorm_quant(x, n_rows, n_in, nullptr, nullptr, 0.0f, false, a, d.s);
+    if (!make_act(d, a, L, x, n_rows)) return -1;
     gemm_epi ep;
     ep.ldy = n_out;
     act_view o;

@@ -176,10 +176,12 @@ def test_matmul_full_m2048_q8_0(jlib, oracle):
     np.testing.assert_array_equal(host(y).view(np.uint32), want.view(np.uint32))
 
 
-@pytest.mark.parametrize("M,N,K", [(1, 128, 8), (31, 128, 40), (33, 96, 128), (64, 36, 136), (197, 384, 768), (40, 1280, 584)])
+@pytest.mark.parametrize("M,N,K", [(1, 128, 8), (31, 128, 40), (33, 96, 128), (64, 36, 136), (197, 384, 768), (40, 1280, 584),
+                                   (40, 1280, 588), (7, 64, 5), (3, 32, 2500)])
 def test_matmul_f32(jlib, M, N, K):
     """f32 weights on the f32 matrix instruction (32 x 32 tiles, K in chunks of 16 columns dealt to eight waves,
-    four accumulators each): ragged rows, features and column chunks, waves without a chunk. Against 64 bits,
+    four accumulators each): ragged rows, features and column chunks (588 are the inputs of a 14 x 14 patch), unaligned
+    rows, waves without a chunk. Against 64 bits,
     within the bound of its sums: at most n roundings on the way of any product, each 2^-24 of the sum of the
     products' magnitudes at most; n = the products of one accumulator (4 per chunk of a wave), then 2 + 7
     additions and the bias."""
