@@ -1,5 +1,7 @@
-// attention.hip - flash attention forward on gfx950 (f16 MFMA, f32 softmax): head width 64 (and 32
-// stored 64 wide) in the LDS-staged kernel below, other multiples of 16 up to 128 in k_attn_any.
+// attention.hip - flash attention forward on gfx950 (f16 MFMA, f32 softmax): head width 64 over more than
+// ATTN_FEW_KEYS keys (and 32 stored 64 wide) in k_attn_hd64, described here; 64 over fewer keys and other
+// multiples of 16 up to 128 in k_attn_any (64 queries per workgroup, its key halves merged at the end, so its
+// results differ from k_attn_hd64's in their last bits).
 //
 // Computes softmax(Q K^T * scale) V per (item, head): the ggml_flash_attn_ext of reference
 // src/jepa.cpp:416-442 (no mask, K/V in f16 as the reference's ggml_cast does, f32 softmax and f32

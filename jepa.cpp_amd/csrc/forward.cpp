@@ -518,7 +518,7 @@ int64_t encode_host(jepa_context * ctx, const jepa_input * in, float * out_host,
     const size_t n_out = (size_t) n_items * R * m->hp.enc.embed_dim;
     if ((int64_t) n_out > out_cap) return -1;
     if (hipSetDevice(ctx->device) != hipSuccess) return -1;
-    // persistent I/O buffers: stable pointers let the captured graph be replayed call after call
+    // device copies of the input and the output, kept between calls
     std::unique_lock<std::recursive_mutex> lk(jepa_hip_mutex());
     if (ctx->io_in_cap < n_in * 4) {
         if (ctx->io_in) hipFree(ctx->io_in);

@@ -89,7 +89,7 @@ __device__ __forceinline__ void stage_barrier() {
 
 // Workgroup tile geometry. WN x WM waves (8: two per SIMD, so one wave's MFMAs fill the other's
 // barrier, LDS-latency and VALU phases, and eight waves keep enough HBM->LDS copies in flight: a wave
-// sustains only ~10 GB/s of loads), each owning TI x TJ MFMA tiles of 32 x 32. The workgroup tile is
+// sustains only ~10 GB/s of loads; the 64x64 tile of few rows has 4, one per SIMD), each owning TI x TJ MFMA tiles of 32 x 32. The workgroup tile is
 // BN = 32 WN TI weight rows by BM = 32 WM TJ tokens. One LDS stage holds 128 B of every one of the
 // BN + BM rows, 16-byte chunks swizzled by lds_slot(): KC = 128 K-columns of int8
 // codes (q8_0 / q4_0, plus the four f16 block scales of every row) or 64 K-columns of f16 values
@@ -1311,12 +1311,13 @@ __global__ __launch_bounds__(64 * WN * WM, 1) void k_gemm_mfma(const void * pA, 
 }
 
 struct tile_cfg { int wn, wm, ti, tj; };
-// Workgroup tiles (BN x BM). The last, 64x64 of four waves (one per SIMD, so less per CU and second than two would
-// do), has the efficiency at which the rule takes it where it means one round of more workgroups and the
-// 128x64 tile would leave CUs idle: us for 128x64 / 64x64, q8_0 576 x 768 x 3072 20.5 / 17.7, 2048 x 384 x 1536
-// 12.4 / 11.0, 1024 x 1024 x 1024 10.3 / 9.1, but 4608 x 768 x 768 14.2 (128x128) / 16.7. Eight-wave tiles: 256x128, 192x128, 128x128 (two wave shapes), 64x128, 128x64,
+// Workgroup tiles (BN x BM) of eight waves: 256x128, 192x128, 128x128 (two wave shapes), 64x128, 128x64,
 // 256x64 (two wave shapes; the second, one weight tile and two token tiles per wave, only for the
-// 256-feature q8_K epilogue)
+// 256-feature q8_K epilogue), 384x64. The last, 64x64 of four waves (one per SIMD, so less per CU and second than
+// two would do), is for few rows: its efficiency is set so that a launch of at most one such tile per CU takes it,
+// and one of several rounds where they come to less work than the other tiles' whole rounds. us for 128x64 / 64x64,
+// q8_0 576 x 768 x 3072 20.5 / 17.7, 2048 x 384 x 1536 12.4 / 11.0, 1024 x 1024 x 1024 10.3 / 9.1, but 4608 x 768 x
+// 768 14.2 (128x128) / 16.7.
 constexpr tile_cfg k_tiles[] = {{4, 2, 2, 2}, {2, 4, 3, 1}, {2, 4, 2, 1}, {4, 2, 1, 2}, {2, 4, 1, 1}, {4, 2, 1, 1}, {4, 2, 2, 1},
                                 {8, 1, 1, 2}, {4, 2, 3, 1}, {2, 2, 1, 1}};
 constexpr int FORCEABLE_TILES = 9;   // the hook's indices; the 64x64 tile runs by the rule alone
@@ -1339,8 +1340,8 @@ int cu_count() {
     return n;
 }
 
-// 4-bit weights (q4_K, packed q4_0) run the tiles whose weight rows pair up into whole 1 KB copies (BN
-// a multiple of 128); q4_K, whose four accumulator sets per MFMA tile must fit 256 VGPRs with two waves
+// 4-bit weights (q4_K, packed q4_0) run the tiles whose weight rows pair up into a whole number of 1 KB copies per
+// wave: BN a multiple of 128, or 64 with four waves; q4_K, whose four accumulator sets per MFMA tile must fit 256 VGPRs with two waves
 // per SIMD, at most two MFMA tiles per wave. The 384x64 tile (for N = 3072: 256 tiles at M = 2048, the
 // role the 192x128 tile has for int8 weights) fits three LDS stages only with 4-bit weights.
 bool tile_ok(int wf, int c) {
@@ -1436,9 +1437,9 @@ void launch_tiles(int c, const kargs & a, hipStream_t s) {
 }
 
 // K parts of an f16-weight GEMM whose tiles leave most CUs idle (the residual GEMMs of a ViT-S/16 image:
-// 197 tokens x 384 outputs are 12 tiles of 128x64, and fc2's K = 1536 is 24 stages per tile, copied at
+// 197 tokens x 384 outputs are 24 tiles of 64x64, and fc2's K = 1536 is 24 stages per tile, copied at
 // the ~80 GB/s one CU's copies sustain). Each of the S parts covers whole 64-column stages. Measured at
-// 197 rows (us, S = 1 / 2 / 3 / 4): K 1536 12.4 / 10.6 / 9.7 / 9.4, K 3072 (N 768) 21.0 / 15.3 / 12.8 /
+// 197 rows with 128x64 tiles (us, S = 1 / 2 / 3 / 4): K 1536 12.4 / 10.6 / 9.7 / 9.4, K 3072 (N 768) 21.0 / 15.3 / 12.8 /
 // 11.9, K 384 6.3 / 7.6 / 7.7 / -, K 768 (N 768) 8.4 / 8.8 / 8.6 / 8.8: the exchange (partial stores, the
 // arrival atomic, the last part's loads) costs ~2 us, so only K >= 1024 (16 stages) splits, into the
 // largest S of 4, 3, 2 that leaves each part 4 stages and each workgroup its own CU. The summation order

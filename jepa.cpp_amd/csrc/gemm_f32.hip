@@ -23,10 +23,12 @@ namespace {
 // columns 8 j + 4 g .. + 3 of its row for step j; the MFMA pairs columns e and 4 + e), one pair of steps
 // ahead; the lines a load leaves half read are finished by the next one out of L1. Each of the four MFMAs
 // of a step has its own accumulator: no chain from one to the next, and sums of K / 32 terms.
-// Measured (us per launch, tokens x features x K): 196 x 384 x 768 11.4 -> 9.5, 256 x 1280 x 584 27.9 ->
-// 13.4, 1024 x 1280 x 584 88.5 -> 36.4 (42 TFLOP/s; the fma rate alone would take 10: half-used lines
-// and 32 rows per load bound it), 2048 x 1024 x 1024 214.6 -> 78.7; relative error against 64 bits
-// 1.36e-7 -> 1.04e-7 at K = 584 (32 partial sums per output instead of 16).
+// Measured against 16 x 32 tiles of VALU fmas (us per launch, tokens x features x K): 196 x 384 x 768 11.4 -> 9.5,
+// 256 x 1280 x 588 27.8 -> 13.8, 1024 x 1280 x 588 88.5 -> 36.8 (42 TFLOP/s; the fma rate alone would take 10:
+// half-used lines and 32 rows per load bound it), 2048 x 1024 x 1024 218 -> 75.7, one row of 384 x 384 7.2 -> 5.6;
+// relative error against 64 bits 1.46e-7 -> 1.12e-7 at K = 768, 1.36e-7 (K = 584) -> 1.05e-7 (588): 32 partial sums
+// per output instead of 16. The sums' order is another one than the fmas', so f32 results differ in their last bits
+// from that kernel's.
 constexpr int F32_KS = 8;
 
 template <int EPI>

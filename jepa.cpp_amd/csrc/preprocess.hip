@@ -149,6 +149,9 @@ __device__ __forceinline__ int16_t tile_tap(const axis_filter & f, double unit, 
 // table uploads took 61 us of kernels, most of it in three byte loads per tap and 11.8 MB of
 // intermediate written and read back (22 MB in and 12.6 MB out would take 4.5 us at the card's copy rate:
 // the taps' VALU work and the latency of each row's loads bound it now).
+// tile_tap sums an output's weights again for each of its taps: ~1 us of those 19, more where an output has more
+// taps, and still ahead of the two kernels at the largest reduction a tile holds (whole calls: four frames of 2160
+// x 3840 to 192, bicubic with 46 taps, 220 us against 625).
 template <int NC>
 __global__ __launch_bounds__(256) void k_resize_tile(const uint8_t * __restrict__ src, float * __restrict__ out, int n, int h, int w,
                                                      int crop, int oy, int ox, int tx, int ty, axis_filter fx, axis_filter fy, int xshift,
